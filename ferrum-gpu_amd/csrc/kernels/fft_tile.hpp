@@ -76,6 +76,23 @@ struct TileLayout {
     }
 };
 
+// LDS layout of a row-wise tile (ROWWISE below), [row][position]: one pad slot
+// per 16 positions and a row pitch of 32/G more (odd from 32 rows up).  A row
+// is loaded by T consecutive lanes and stored by lanes along the rows, so the
+// first scatter runs along positions and every gather across rows; with this
+// pitch a model of 64 four-byte banks serving 32 lanes of an 8-byte access
+// per cycle has no conflicts beyond two lanes per bank in the scatter of T < 32.
+template <int LOGP, int G>
+struct RowTileLayout {
+    static constexpr int N = 1 << LOGP;
+    static constexpr int P = N + N / 16 + (G >= 32 ? 1 : 32 / G);
+    static constexpr int ELEMS = P * G;
+    __device__ __forceinline__ static int at(int pos, int c) { return c * P + lds_pos<>(pos); }
+    // at(t + d, c) - at(t, c) for t < T and d a multiple of T, T a multiple
+    // or a divisor of 16 (t never carries into the next pad).
+    __device__ __forceinline__ static constexpr int off(int d) { return d + d / 16; }
+};
+
 // Stockham stages on a [position][column] LDS tile: thread (c, q) holds
 // positions q + T*m of column c.  LDS addresses are a per-thread base plus
 // compile-time offsets (ds_read / ds_write immediates) wherever the layout
@@ -124,6 +141,47 @@ struct TileStages {
     }
 };
 
+// The 16-element row tiles that load directly: 16 rows or more (128 points).
+// Measured on gfx950, us per execution against the staged form: 2^21 at 16
+// MiB 30.4 -> 29.5, at 112 MiB 114.8 -> 114.1, at 512 MiB 483.8 -> 483.3.
+// The 8-row tile of 512 points lost at 120 MiB (2^17 84.0 -> 84.9).
+template <int G>
+constexpr bool row_tile_direct() { return G >= 16; }
+
+// The same stages on a [row][position] LDS tile.  Stage 0 (radix 16, no
+// twiddles) ran on the positions the thread loaded, t0 + T*m of row c0; its
+// scatter goes to that row, and every gather takes the positions t + T*m of
+// row c, so the exchange also turns the tile (lanes along the rows).
+template <int LOGL, int LOGE, int G, int S>
+struct RowTileStages {
+    using Sh = StockhamShape<LOGL, LOGE>;
+    using Lay = RowTileLayout<LOGL, G>;
+    __device__ __forceinline__ static void run(float2* x, int cs, int ts, int c, int t,
+                                               const float2* __restrict__ tw, float2* __restrict__ lds) {
+        stockham_stage_regs<LOGL, LOGE, S>(x, t, tw);
+        if constexpr (S + 1 < Sh::NSTAGES) {
+            static_assert(LOGE == 4 && S < Sh::NFULL, "exchanges follow radix-16 stages");
+            static_assert(Sh::T % 16 == 0 || 16 % Sh::T == 0, "RowTileLayout::off");
+            constexpr int L = 1 << (S * LOGE);
+            if constexpr (S > 0) __syncthreads();  // previous readers of the tile are done
+            if constexpr (L == 1) {
+                float2* base = lds + cs * Lay::P + 17 * ts;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) base[r] = x[r];
+            } else {
+                float2* base = lds + Lay::at(stockham_dst<LOGL, LOGE, S>(ts, 0, 0), cs);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) base[r * (L + L / 16)] = x[r];
+            }
+            __syncthreads();
+            const float2* base = lds + Lay::at(t, c);
+#pragma unroll
+            for (int m = 0; m < Sh::E; ++m) x[m] = base[Lay::off(Sh::T * m)];
+            RowTileStages<LOGL, LOGE, G, S + 1>::run(x, c, t, c, t, tw, lds);
+        }
+    }
+};
+
 // This workgroup's tile: its (t0, t1) indices and input / output bases.
 struct TileCoords {
     uint32_t t0, t1;
@@ -157,9 +215,12 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 }
 
 // ROWWISE: input elements of a column are contiguous (ies == 1, rows of a
-// matrix), so loads run along elements and the tile is transposed into LDS
-// first; otherwise columns are contiguous (ics == 1) and each thread loads its
-// own Stockham positions straight into VGPRs.  Output always has ocs == 1.
+// matrix).  Row tiles that row_tile_direct names load a row's Stockham
+// positions t0 + T*m with T consecutive lanes (8*T contiguous bytes per
+// access) and the first exchange turns the tile (RowTileStages); the others
+// load along the rows and turn the tile through LDS first.  Otherwise
+// columns are contiguous (ics == 1) and consecutive lanes load consecutive
+// columns.  Output always has ocs == 1.
 // LOAD_CACHED / STORE_CACHED select the pass's cache policy (gload/gstore).
 // CONJ: the body reads the inverse's conjugation flags; forward passes
 // (flags == 0) run the CONJ = false body, which has no per-element selects.
@@ -172,9 +233,6 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g, float2* __restrict__ lds) {
     using Sh = StockhamShape<LOGL, LOGE>;
-    using Lay = TileLayout<LOGL, G>;
-    constexpr int THREADS = G * Sh::T;
-
     const int tid = threadIdx.x;
     const int c = tid % G;
     const int q = tid / G;
@@ -184,7 +242,16 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
     char* out_tile = reinterpret_cast<char*>(out + tc.ob);
 
     float2 x[Sh::E];
-    if constexpr (ROWWISE) {
+    constexpr bool DIRECT = ROWWISE && row_tile_direct<G>();
+    const int c0 = DIRECT ? tid / Sh::T : c, q0 = DIRECT ? tid % Sh::T : q;
+    if constexpr (DIRECT) {
+        const char* row = in_tile + (uint32_t)((c0 * g.ics + q0) * sizeof(float2));
+#pragma unroll
+        for (int m = 0; m < Sh::E; ++m)
+            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(row) + Sh::T * m);
+    } else if constexpr (ROWWISE) {
+        using Lay = TileLayout<LOGL, G>;
+        constexpr int THREADS = G * Sh::T;
         // Coalesced along each row: linear element li -> (column li / L, position li % L).
 #pragma unroll
         for (int m = 0; m < Sh::E; ++m) {
@@ -216,7 +283,8 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
             for (int m = 0; m < Sh::E; ++m) x[m] = cconj(x[m]);
         }
     }
-    TileStages<LOGL, LOGE, G, 0>::run(x, q, c, tw, lds);
+    if constexpr (DIRECT) RowTileStages<LOGL, LOGE, G, 0>::run(x, c0, q0, c, q, tw, lds);
+    else TileStages<LOGL, LOGE, G, 0>::run(x, q, c, tw, lds);
 
     if (g.log_m != 0) {
         const uint64_t r = (uint64_t)g.twc * c + (uint64_t)g.tw0 * t0 + (uint64_t)g.tw1 * t1;
@@ -304,6 +372,60 @@ struct HalvesStages {
     }
 };
 
+// Whether the row-wise tile loads its Stockham positions directly (T = L/32
+// consecutive lanes per row, 8 T contiguous bytes) and turns the tile in the
+// first exchange, instead of loading along the rows and turning it through
+// two LDS rounds of its own: from 512 points up.  Measured on gfx950 at 512
+// MiB per execution, us, six alternations against the staged form: 2^17 (512
+// points) 332.2 -> 328.2, 2^18 342.9 -> 335.3, 2^19 364.6 -> 354.5, 2^20
+// 369.4 -> 363.5 (1024 points); at 32 MiB 2^18 36.0 -> 34.2.  At 256 points
+// (64-byte pieces, every row of the tile at one L2 channel) it lost: 2^16
+// 322.2 -> 327.1, one 2^24 127.4 -> 130.3, and with 16-byte loads (128-byte
+// pieces) 321.7 -> 325.7, 127.1 -> 129.0.
+template <int LOGL>
+constexpr bool row_halves_direct() { return LOGL >= 9; }
+
+// The same stages on a [row][position] tile of L/2 positions: every
+// exchange's round h scatters to row cs (stage 0: the row the thread loaded)
+// and gathers row c (RowTileLayout).
+template <int LOGL, int S, int G>
+struct RowHalvesTileStages {
+    __device__ __forceinline__ static void run(float2* x, float2* y, int cs, int ts, int c, int t,
+                                               const float2* __restrict__ tw, float2* __restrict__ lds) {
+        using H = HalvesShape<LOGL>;
+        using St = HalvesStage<LOGL, S>;
+        halves_stage<LOGL, S>(x, y, ts, tw);
+        if constexpr (S + 1 < H::NSTAGES) {
+            using Lay = RowTileLayout<LOGL - 1, G>;
+            static_assert(St::R == 16 && (H::T % 16 == 0 || 16 % H::T == 0), "exchanges follow radix-16 stages");
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (S > 0 || h > 0) __syncthreads();  // the previous round's readers are done
+#pragma unroll
+                for (int ii = 0; ii < St::NB / 2; ++ii) {
+                    const int i = h * (St::NB / 2) + ii;
+                    const int b = ts + H::T * i;
+                    if constexpr (St::L == 1) {
+                        float2* base = lds + cs * Lay::P + 17 * (b - (H::HALF / 16) * h);
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) base[q] = y[i + St::NB * q];
+                    } else {
+                        const int d0 = (b >> (4 * S)) * St::L * 16 + (b & (St::L - 1)) - H::HALF * h;
+                        float2* base = lds + Lay::at(d0, cs);
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) base[q * (St::L + St::L / 16)] = y[i + St::NB * q];
+                    }
+                }
+                __syncthreads();
+                const float2* base = lds + Lay::at(t, c);
+#pragma unroll
+                for (int m = 0; m < H::E / 2; ++m) x[(H::E / 2) * h + m] = base[Lay::off(H::T * m)];
+            }
+            RowHalvesTileStages<LOGL, S + 1, G>::run(x, y, c, t, c, t, tw, lds);
+        }
+    }
+};
+
 template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool CONJ, bool ROWWISE>
 __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ in, float2* __restrict__ out,
                                                      const float2* __restrict__ tw, const float2* __restrict__ big,
@@ -316,8 +438,17 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
     const char* in_tile = reinterpret_cast<const char*>(in + tc.ib);
     char* out_tile = reinterpret_cast<char*>(out + tc.ob);
 
+    constexpr bool DIRECT = ROWWISE && row_halves_direct<LOGL>();
     float2 x[H::E], y[H::E];
-    if constexpr (ROWWISE) {
+    const int c0 = DIRECT ? tid / H::T : c, t0 = DIRECT ? tid % H::T : t;
+    if constexpr (DIRECT) {
+        // Rows contiguous (ies == 1): T consecutive lanes load positions
+        // t0 + T m of row c0, every load of the tile issued at once.
+        const char* row = in_tile + (uint32_t)((c0 * g.ics + t0) * sizeof(float2));
+#pragma unroll
+        for (int m = 0; m < H::E; ++m)
+            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(row) + H::T * m);
+    } else if constexpr (ROWWISE) {
         // Rows contiguous (ies == 1): every load of the tile is issued at
         // once, coalesced along the rows (y[m]: half m / (E/2) of the
         // positions, linear element li -> row li / HALF, position li % HALF),
@@ -362,7 +493,8 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
             for (int m = 0; m < H::E; ++m) x[m] = cconj(x[m]);
         }
     }
-    HalvesStages<LOGL, 0, G>::run(x, y, t, c, tw, lds);
+    if constexpr (DIRECT) RowHalvesTileStages<LOGL, 0, G>::run(x, y, c0, t0, c, t, tw, lds);
+    else HalvesStages<LOGL, 0, G>::run(x, y, t, c, tw, lds);
     if (g.log_m != 0) {
         // Four-step twiddle W^(r*(t + T*m)) by one 32-step recurrence (about
         // 2e-6 relative at its end, 1e-4 is the gate); restarting it at m = 16,
@@ -388,7 +520,8 @@ template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool ROWWISE = f
 __device__ __forceinline__ void fft_tile_halves_pass(const float2* __restrict__ in, float2* __restrict__ out,
                                                      const float2* __restrict__ tw, const float2* __restrict__ big,
                                                      const TileGeom& g) {
-    __shared__ float2 lds[TileLayout<LOGL - 1, G>::ELEMS];
+    __shared__ float2 lds[ROWWISE && row_halves_direct<LOGL>() ? RowTileLayout<LOGL - 1, G>::ELEMS
+                                                                : TileLayout<LOGL - 1, G>::ELEMS];
     if (g.flags)
         fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, true, ROWWISE>(in, out, tw, big, g, lds);
     else
@@ -400,7 +533,7 @@ template <int LOGL, int LOGE, int G, bool ROWWISE, bool TWREC, bool LOAD_CACHED,
 __device__ __forceinline__ void fft_tile_pass(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g) {
-    __shared__ float2 lds[TileLayout<LOGL, G>::ELEMS];
+    __shared__ float2 lds[ROWWISE && row_tile_direct<G>() ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
     if (g.flags)
         fft_tile_body<LOGL, LOGE, G, ROWWISE, TWREC, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
     else
