@@ -248,6 +248,36 @@ bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise) {
     return (g == 16 && (log_l == 9 || log_l == 10)) || (g == 32 && log_l == 8);
 }
 
+uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
+    // A launch in the pass's own tiles of G columns that would leave CUs idle,
+    // or hold them at less than one round of narrower tiles, takes the
+    // narrowest form (fft_tile_narrow; at least one wave per workgroup) whose
+    // workgroups are resident all at once: 1024 threads per CU (16 waves at
+    // the kernels' 128 VGPRs; the LDS allows as many), so 1024 / block of the
+    // pass's own blocks, which a narrow form of half the elements per thread
+    // equals per column; 4 columns, whose 32-byte pieces cost L2 requests,
+    // only up to one workgroup per CU.  Measured on gfx950, us per
+    // execution, own tiles / narrow by this rule (the passes of one plan
+    // narrowed one at a time: 4, 8, 16 columns): first pass of 256 points,
+    // 2^16 x 1 12.4 / 10.0 (8 columns 10.3), x 16 17.0 / 14.6 at 8, x 48 27.8
+    // / 22.0 at 16 (8: 25.1), x 64 31.8 / 24.4 at 16 (8: 29.2); past one round
+    // own tiles are no worse (x 96, loading through the caches: 33.5, 16
+    // columns 34.1).  1024 points: 2^20 x 1 25.8 / 20.4 at 4 or 8, x 4 37.9 /
+    // 31.1 at 8, x 8 (two rounds) 49.6 / 52.8.  2D columns: 256 x 256 x 1 8.5
+    // / 7.7, x 64 25.8 / 24.0 at 16 (8: 27.2), 1024 x 1024 x 3 24.2 / 23.2,
+    // x 8 (two rounds) 48.2 / 50.9; 4096 x 64 21.9 / 16.6.  Whole plans:
+    // 2^16 x 1 12.4 -> 6.9, 2^18 x 16 35.6 -> 26.1, 2^20 x 1 25.8 -> 16.3.
+    // Not with two chunks in flight, where the other stream's launch fills the
+    // CUs: 2^16 x 300 (a last chunk of 44 transforms) 104.3 -> 107.4.
+    if (log_l == 8 && g == 16) return 0;  // the middle pass of 2^23 points and more (tile_narrows)
+    const uint64_t resident = (uint64_t)cu_count * (1024 / (g * ((1u << log_l) / 32)));
+    for (uint32_t w = 4; w < g && w <= 16; w *= 2) {
+        if ((w << log_l) / 16 < 64) continue;
+        if (tiles * (g / w) <= (w == 4 ? (uint64_t)cu_count : resident)) return w;
+    }
+    return 0;
+}
+
 bool split_2d_columns(uint32_t log_rows) { return log_rows > 12; }
 
 namespace {
@@ -403,6 +433,9 @@ void FftPlan::add_tile(const HipBackend::Module& mod, uint32_t log_l, uint32_t g
     s.src = src;
     s.dst = dst;
     s.tw = stage_table(log_l, elems_per_thread_log(log_l));
+    s.halves = halves || row_halves;
+    s.log_l = log_l;
+    s.width = g;
     s.geom = geom;
     s.per_unit = tiles_per_unit;
     steps_.push_back(s);
@@ -534,6 +567,18 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         t.ocs = 1;
         t.oes = N / L;
         p->add_tile(mod, log_l, g, true, t, (uint64_t)t.t0n * t.t1n, Buf::Work, Buf::Out, p->policy(P - 1, P));
+        // A plan of one chunk whose input, workspace and output fit the
+        // Infinity Cache together loads its input through it (the caller has
+        // often just written it; a streamed load neither fills the cache nor
+        // is served at its rate).  Measured on gfx950 over three alternating
+        // input / output pairs, us per execution, streamed / cached loads: 48
+        // MiB 2^16 38.3 / 33.5, 2^18 42.9 / 38.5, 2^20 46.2 / 41.6; 64 MiB
+        // 45.9 / 42.0, 49.3 / 46.0, 53.6 / 49.6, 2^23 67.1 / 62.5; 96 MiB 68.0
+        // / 67.4, 75.8 / 71.4, 79.6 / 75.7; 128 MiB 2^16 86.5 / 88.8, 2^24
+        // 128.2 / 131.2.  The 8-row last pass of 512 points stores through
+        // the caches too: 2^17 32 MiB 28.1 / 27.7, 64 MiB 46.0 / 53.4.
+        const uint64_t bytes = 8ull * N * batch;
+        p->load_cached_ = p->cached_ && p->chunks() == 1 && bytes <= (g < 16 ? 32ull << 20 : 96ull << 20);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -741,6 +786,7 @@ void FftPlan::exec(const void* in, void* out, Direction dir, bool normalize, hip
     const float scale = scale_for(dir, normalize);
     const void* big = big_.data();
     const uint64_t unit = elems();
+    const int cu_count = dev_->handle()->cu_count;
     const hipStream_t main = stream ? stream : HipBackend::default_stream(dev_->handle());
     const std::vector<Step>& steps = (in == out && !steps_in_place_.empty()) ? steps_in_place_ : steps_;
     bool two = streams() == 2;
@@ -809,14 +855,30 @@ void FftPlan::exec(const void* in, void* out, Direction dir, bool normalize, hip
                 TileGeom g = s.geom;
                 g.flags = flags;
                 g.scale = scale;
-                const uint64_t tiles = s.per_unit * units;
-                g.remap = (s.tile_order != 0 && tiles % s.order_unit == 0) ? s.tile_order : 0u;
+                uint64_t tiles = s.per_unit * units;
+                uint32_t order = s.tile_order, order_unit = s.order_unit;
+                Dim3 block = s.block;
+                if (const uint32_t w = s.halves && !two ? narrow_width(s.log_l, s.width, tiles, cu_count) : 0) {
+                    const uint32_t k = s.width / w;  // the geometry steps tiles by the width (add_tile)
+                    tiles *= k;
+                    g.t0n *= k;
+                    g.is0 /= k;
+                    g.os0 /= k;
+                    g.tw0 /= k;
+                    g.flags |= w << FG_PASS_WIDTH_SHIFT;
+                    block = Dim3((w << s.log_l) / 16);
+                    order = w < 16 ? FG_TILE_ORDER_LINE_GROUPS : 0u;
+                    order_unit = w < 16 ? 8 * (16 / w) : 1;
+                } else if (i == 0 && load_cached_) {
+                    g.flags |= FG_PASS_LOAD_CACHED;
+                }
+                g.remap = (order != 0 && tiles % order_unit == 0) ? order : 0u;
                 void* args[] = {&src, &dst, (void*)&tw, (void*)&big, &g};
-                const Dim3 grid((uint32_t)(s.per_unit * units));
+                const Dim3 grid((uint32_t)tiles);
                 if (events)
-                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, s.block, 0, args, events[launch]);
+                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, block, 0, args, events[launch]);
                 else
-                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, s.block, 0, args);
+                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, block, 0, args);
             }
             ++launch;
         }

@@ -145,6 +145,8 @@ private:
         uint64_t per_unit = 0;
         uint32_t tile_order = 0;                // tile: TileGeom::remap (FG_TILE_ORDER_*) when the grid
         uint32_t order_unit = 1;                // is a multiple of order_unit, else the natural order
+        bool halves = false;                    // tile: 32 elements per thread, so narrow_width applies
+        uint32_t log_l = 0, width = 0;          // tile: log2 of the pass's length, columns per workgroup
         TileGeom geom{};                        // tile: addressing (flags/scale/remap set at exec)
     };
 
@@ -202,6 +204,7 @@ private:
     size_t batch_;
     size_t chunk_;         // units per chunk (batch_ when not chunked)
     bool cached_ = false;  // intermediates kept cached (else every pass streams)
+    bool load_cached_ = false;  // 1D: the first pass loads its input through the caches too
     std::vector<Step> steps_;
     std::vector<Step> steps_in_place_;  // when not empty: the passes of in-place executions (in == out)
     std::vector<std::pair<uint32_t, Buffer<Cf32, HipBackend>>> stage_tables_;
@@ -250,6 +253,9 @@ bool use_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
 // exchanges in halves (fg_tile_l*_g*_rh): 32-row tiles of 256 points, 16-row
 // tiles of 512 / 1024 points.
 bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
+// Columns per workgroup of a launch of `tiles` tiles of a halves pass (2^log_l
+// points, g columns per tile) in its narrow form; 0: its own tiles.
+uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count);
 // Whether the column FFT of an image with 2^log_rows rows runs as two passes.
 bool split_2d_columns(uint32_t log_rows);
 // Largest chunk (bytes of one chunk's array) a multi-launch plan created from

@@ -355,7 +355,7 @@ extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
         fg_tile_l##LOGL##_g##G##_##TAG(const float2* __restrict__ in, float2* __restrict__ out,     \
                                        const float2* __restrict__ tw, const float2* __restrict__ big, \
                                        TileGeom g) {                                                  \
-        fft_tile_pass<LOGL, (LOGL < 4 ? LOGL : 4), G, RW, true, LC, SC>(in, out, tw, big, g);        \
+        fft_tile_pass<LOGL, (LOGL < 4 ? LOGL : 4), G, RW, LC, SC>(in, out, tw, big, g);        \
     }
 #define FG_TILE(LOGL, G, RW, TAG)                  \
     FG_TILE_P(LOGL, G, RW, TAG, false, false)      \

@@ -30,25 +30,32 @@ __device__ __forceinline__ float2 big_twiddle(const float2* __restrict__ big, ui
     return cmul(big[ep >> 12], big[4096 + (ep & 4095)]);
 }
 
-// Multiplies x[m] (output position k = q + T*m) by W_M^(r*k).  TWREC = false
-// looks every factor up (2 table reads + 1 multiply each); TWREC = true looks
-// up W^(r*q) and W^(r*T) once and forms the rest as W^(r*q) * (W^(r*T))^m by
-// repeated multiplication (error grows by about one rounding per step, ~1e-6
-// relative after 16 steps).
-template <int E, int T, bool TWREC>
+// Multiplies x[m] (output position k = q + T*m) by W_M^(r*k), formed as
+// W^(r*q) * (W^(r*T))^m by repeated multiplication from two looked-up factors
+// (error grows by about one rounding per step, ~1e-6 relative after 16
+// steps).  HALVES (E = 16): the recurrence of the 32-element kernels, which
+// steps by T/2 from position q mod T/2, so that both forms of a pass give the
+// same bits; the thread's positions are every second one of its 32.
+template <int E, int T, bool HALVES = false>
 __device__ __forceinline__ void apply_pass_twiddle(float2* x, const float2* __restrict__ big, uint64_t r, int q,
                                                    uint32_t log_m) {
-    if constexpr (TWREC) {
-        float2 w = big_twiddle(big, r * (uint64_t)q, log_m);
-        const float2 step = big_twiddle(big, r * (uint64_t)T, log_m);
+    constexpr int STEP = HALVES ? T / 2 : T;
+    float2 w = big_twiddle(big, r * (uint64_t)(HALVES ? q % STEP : q), log_m);
+    const float2 step = big_twiddle(big, r * (uint64_t)STEP, log_m);
+    if constexpr (HALVES) {
+        const bool odd = q >= STEP;
+#pragma unroll
+        for (int m = 0; m < E; ++m) {
+            const float2 w1 = cmul(w, step);
+            x[m] = cmul(x[m], odd ? w1 : w);
+            if (m + 1 < E) w = cmul(w1, step);
+        }
+    } else {
 #pragma unroll
         for (int m = 0; m < E; ++m) {
             x[m] = cmul(x[m], w);
             if (m + 1 < E) w = cmul(w, step);
         }
-    } else {
-#pragma unroll
-        for (int m = 0; m < E; ++m) x[m] = cmul(x[m], big_twiddle(big, r * (uint64_t)(q + T * m), log_m));
     }
 }
 
@@ -228,7 +235,8 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 // 32-bit per-lane byte offset, so each access costs no 64-bit vector
 // arithmetic; a tile's offsets stay below 2^32 bytes (one transform or image
 // spans at most 128 MiB).
-template <int LOGL, int LOGE, int G, bool ROWWISE, bool TWREC, bool LOAD_CACHED, bool STORE_CACHED, bool CONJ>
+template <int LOGL, int LOGE, int G, bool ROWWISE, bool DIRECT, bool HALVES_TW, bool LOAD_CACHED, bool STORE_CACHED,
+          bool CONJ>
 __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g, float2* __restrict__ lds) {
@@ -242,7 +250,7 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
     char* out_tile = reinterpret_cast<char*>(out + tc.ob);
 
     float2 x[Sh::E];
-    constexpr bool DIRECT = ROWWISE && row_tile_direct<G>();
+    static_assert(ROWWISE || !DIRECT, "DIRECT is a way to load rows");
     const int c0 = DIRECT ? tid / Sh::T : c, q0 = DIRECT ? tid % Sh::T : q;
     if constexpr (DIRECT) {
         const char* row = in_tile + (uint32_t)((c0 * g.ics + q0) * sizeof(float2));
@@ -288,7 +296,7 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
 
     if (g.log_m != 0) {
         const uint64_t r = (uint64_t)g.twc * c + (uint64_t)g.tw0 * t0 + (uint64_t)g.tw1 * t1;
-        apply_pass_twiddle<Sh::E, Sh::T, TWREC>(x, big, r, q, g.log_m);
+        apply_pass_twiddle<Sh::E, Sh::T, HALVES_TW>(x, big, r, q, g.log_m);
     }
     const uint32_t lane_off = (uint32_t)((c + (uint64_t)q * g.oes) * sizeof(float2));
     const uint64_t row_step = (uint64_t)Sh::T * g.oes * sizeof(float2);
@@ -501,7 +509,7 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
         // from two more table reads or from four squarings of the step,
         // measured 1.7-2.4 us slower per 128 MiB pass.
         const uint64_t r = (uint64_t)g.twc * c + (uint64_t)g.tw0 * tc.t0 + (uint64_t)g.tw1 * tc.t1;
-        apply_pass_twiddle<H::E, H::T, true>(y, big, r, t, g.log_m);
+        apply_pass_twiddle<H::E, H::T>(y, big, r, t, g.log_m);
     }
     const uint32_t lane_off = (uint32_t)((c + (uint64_t)t * g.oes) * sizeof(float2));
     const uint64_t row_step = (uint64_t)H::T * g.oes * sizeof(float2);
@@ -516,28 +524,91 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
     }
 }
 
+// The narrow forms of a halves pass: W < G columns per workgroup of W L/16
+// threads, 16 elements per thread, for launches whose own tiles leave the GPU
+// short of workgroups (the rule and its measurements: narrow_width in
+// fft_plan.cpp).  Twice the threads per column shorten each thread's chain,
+// and the columns of one line group run on one XCD (tile_coords), so its L2
+// joins their 8 W-byte pieces.  Loaded through the caches; stored so too,
+// except row tiles of 16 rows, which write whole 128-byte lines and stream
+// them as the pass's own form does (2^16 x 64, us: 23.8 cached, 23.1
+// streamed; 256 x 256 columns lose: 24.0 -> 24.8).  The same butterflies on
+// the same values and the same twiddle recurrence: every width gives the
+// same bits.
+template <int LOGL, int W, bool ROWWISE, bool STREAM_OUT>
+__device__ __forceinline__ void fft_tile_narrow(const float2* __restrict__ in, float2* __restrict__ out,
+                                                const float2* __restrict__ tw, const float2* __restrict__ big,
+                                                const TileGeom& g, float2* __restrict__ lds) {
+    constexpr bool STORE_CACHED = !(STREAM_OUT && ROWWISE && W >= 16);
+    if (g.flags & FG_PASS_CONJ)
+        fft_tile_body<LOGL, 4, W, ROWWISE, ROWWISE, true, true, STORE_CACHED, true>(in, out, tw, big, g, lds);
+    else
+        fft_tile_body<LOGL, 4, W, ROWWISE, ROWWISE, true, true, STORE_CACHED, false>(in, out, tw, big, g, lds);
+}
+
+// The widths a halves pass can be narrowed to: below its own, at least one
+// wave per workgroup.  The 16-column middle pass of 256 points belongs to
+// plans of 2^23 points and more, whose launches always fill the GPU.
+template <int LOGL, int G, int W>
+constexpr bool tile_narrows() { return W < G && (W << LOGL) / 16 >= 64 && !(LOGL == 8 && G == 16); }
+
+template <int LOGL, int G, bool ROWWISE, int W>
+constexpr int tile_narrow_lds() {
+    if (!tile_narrows<LOGL, G, W>()) return 0;
+    return ROWWISE ? RowTileLayout<LOGL, W>::ELEMS : TileLayout<LOGL, W>::ELEMS;
+}
+
+// LDS of a halves pass: its own tile's, or a narrow form's (at most 3 % more).
+template <int LOGL, int G, bool ROWWISE>
+constexpr int tile_halves_lds() {
+    int n = ROWWISE && row_halves_direct<LOGL>() ? RowTileLayout<LOGL - 1, G>::ELEMS : TileLayout<LOGL - 1, G>::ELEMS;
+    for (int w : {tile_narrow_lds<LOGL, G, ROWWISE, 4>(), tile_narrow_lds<LOGL, G, ROWWISE, 8>(),
+                  tile_narrow_lds<LOGL, G, ROWWISE, 16>()})
+        n = w > n ? w : n;
+    return n;
+}
+
 template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool ROWWISE = false>
 __device__ __forceinline__ void fft_tile_halves_pass(const float2* __restrict__ in, float2* __restrict__ out,
                                                      const float2* __restrict__ tw, const float2* __restrict__ big,
                                                      const TileGeom& g) {
-    __shared__ float2 lds[ROWWISE && row_halves_direct<LOGL>() ? RowTileLayout<LOGL - 1, G>::ELEMS
-                                                                : TileLayout<LOGL - 1, G>::ELEMS];
-    if (g.flags)
+    __shared__ float2 lds[tile_halves_lds<LOGL, G, ROWWISE>()];
+    const uint32_t w = g.flags >> FG_PASS_WIDTH_SHIFT;
+    if constexpr (tile_narrows<LOGL, G, 4>()) {
+        if (w == 4) return fft_tile_narrow<LOGL, 4, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+    }
+    if constexpr (tile_narrows<LOGL, G, 8>()) {
+        if (w == 8) return fft_tile_narrow<LOGL, 8, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+    }
+    if constexpr (tile_narrows<LOGL, G, 16>()) {
+        if (w == 16) return fft_tile_narrow<LOGL, 16, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+    }
+    if constexpr (!LOAD_CACHED && STORE_CACHED) {
+        if (g.flags & FG_PASS_LOAD_CACHED) {
+            if (g.flags & FG_PASS_CONJ)
+                fft_tile_halves_body<LOGL, G, true, true, true, ROWWISE>(in, out, tw, big, g, lds);
+            else
+                fft_tile_halves_body<LOGL, G, true, true, false, ROWWISE>(in, out, tw, big, g, lds);
+            return;
+        }
+    }
+    if (g.flags & FG_PASS_CONJ)
         fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, true, ROWWISE>(in, out, tw, big, g, lds);
     else
         fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, false, ROWWISE>(in, out, tw, big, g, lds);
 }
 
 // One pass: a forward body and one that applies the inverse's conjugations.
-template <int LOGL, int LOGE, int G, bool ROWWISE, bool TWREC, bool LOAD_CACHED, bool STORE_CACHED>
+template <int LOGL, int LOGE, int G, bool ROWWISE, bool LOAD_CACHED, bool STORE_CACHED>
 __device__ __forceinline__ void fft_tile_pass(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g) {
-    __shared__ float2 lds[ROWWISE && row_tile_direct<G>() ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
-    if (g.flags)
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, TWREC, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
+    constexpr bool DIRECT = ROWWISE && row_tile_direct<G>();
+    __shared__ float2 lds[DIRECT ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
+    if (g.flags & FG_PASS_CONJ)
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, DIRECT, false, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
     else
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, TWREC, LOAD_CACHED, STORE_CACHED, false>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, DIRECT, false, LOAD_CACHED, STORE_CACHED, false>(in, out, tw, big, g, lds);
 }
 
 }  // namespace fg

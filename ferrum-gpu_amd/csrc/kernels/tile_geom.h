@@ -13,6 +13,14 @@ namespace fg {
 /* Per-pass flags (Stockham and tile kernels alike). */
 #define FG_PASS_CONJ_IN 1u        /* conjugate every element on load */
 #define FG_PASS_CONJ_SCALE_OUT 2u /* conjugate, then multiply by `scale`, on store */
+#define FG_PASS_CONJ (FG_PASS_CONJ_IN | FG_PASS_CONJ_SCALE_OUT)
+/* Tile passes that stream their input in: load it through the caches instead
+ * (a plan's only chunk, small enough to stay in the Infinity Cache). */
+#define FG_PASS_LOAD_CACHED 4u
+/* Halves tile passes: flags >> FG_PASS_WIDTH_SHIFT is the columns per
+ * workgroup of a launch in the kernel's narrow form (fft_tile_halves_pass),
+ * 0 for its own width. */
+#define FG_PASS_WIDTH_SHIFT 8
 
 /* Tile orders of narrow tiles (G < 16 columns: 128 / (8 G) tiles share each
  * 128-byte line).  Workgroups are dealt round-robin over the 8 XCDs, so
