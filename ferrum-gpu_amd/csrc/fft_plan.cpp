@@ -270,7 +270,7 @@ uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) 
     // Not with two chunks in flight, where the other stream's launch fills the
     // CUs: 2^16 x 300 (a last chunk of 44 transforms) 104.3 -> 107.4.
     if (log_l == 8 && g == 16) return 0;  // the middle pass of 2^23 points and more (tile_narrows)
-    const uint64_t resident = (uint64_t)cu_count * (1024 / (g * ((1u << log_l) / 32)));
+    const uint64_t resident = (uint64_t)cu_count * (1024 / (g * ((1u << log_l) / 32)));  // for w >= 8
     for (uint32_t w = 4; w < g && w <= 16; w *= 2) {
         if ((w << log_l) / 16 < 64) continue;
         if (tiles * (g / w) <= (w == 4 ? (uint64_t)cu_count : resident)) return w;
@@ -324,7 +324,17 @@ size_t chunk_units_for(uint64_t unit_bytes, size_t batch, size_t limit, bool* ca
 bool FftPlan::choose_chunk(bool two_in_flight) {
     const size_t limit = chunk_limit_bytes();
     const uint64_t unit = 8ull * elems();
-    if (two_in_flight && unit <= limit / 2) {
+    // Two chunks in flight from a batch of the limit up.  Below it one chunk
+    // on one stream is faster: the second stream's fork and join cost about 15
+    // us, and the last chunk is a remainder.  Measured on gfx950 under the
+    // 256 MiB limit, us per execution, two chunks / one: 2^16 150 MiB 104.6 /
+    // 101.6, 200 MiB 141.7 / 129.9, 240 MiB 161.6 / 153.1, 2^18 140 MiB 107.3
+    // / 98.8, 240 MiB 173.3 / 158.9, 2^20 208 MiB 171.1 / 158.4, 248 MiB 188.0
+    // / 182.3, 2^22 224 MiB 224.7 / 215.8.  From 512 MiB (two or more chunks
+    // of 256 MiB on one stream) it loses: 2^16 323.3 / 344.5, 2^24 480.8 /
+    // 515.2.
+    const uint64_t all = unit > SIZE_MAX / batch_ ? SIZE_MAX : unit * batch_;
+    if (two_in_flight && all >= limit && unit <= limit / 2) {
         chunk_ = chunk_units_for(unit, batch_, limit / 2, &cached_);
         if (chunks() > 1) return true;
     }
@@ -433,7 +443,8 @@ void FftPlan::add_tile(const HipBackend::Module& mod, uint32_t log_l, uint32_t g
     s.src = src;
     s.dst = dst;
     s.tw = stage_table(log_l, elems_per_thread_log(log_l));
-    s.halves = halves || row_halves;
+    // The 8-row tile of 512 points runs the body the narrow forms run.
+    s.narrows = halves || row_halves || (rowwise && g == 8);
     s.log_l = log_l;
     s.width = g;
     s.geom = geom;
@@ -546,12 +557,12 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         const uint32_t log_l = logs[P - 1];
         const uint64_t L = 1ull << log_l, n1 = 1ull << logs[0];
         uint32_t g = p->cached_ ? cached_tile_columns(log_l, true) : tile_columns(log_l);
-        // With two chunks in flight (below) the 16-row tile wins at 512
-        // points too (measured with the 512-point last digits of earlier
-        // splits, 2^18 = 512 * 512 and 2^19 = 1024 * 512: 397 / 406 us at 512
-        // MiB with 8 rows on one stream -> 370 / 376 us with 16 rows on two);
-        // 2^17 = 256 * 512 takes it now, in halves (use_row_halves_tile).
-        if (two && g < 16) g = 16;
+        // 2^17 = 256 * 512: the 16-row tile (in halves, output streamed) with
+        // two chunks in flight and for one chunk of more than 40 MiB, where
+        // the 8-row tile's cached stores displace the workspace.  Measured on
+        // gfx950, us per execution, 8 rows / 16: 48 MiB 36.1 / 33.9, 64 MiB
+        // 47.4 / 41.7, 150 MiB 114.8 / 103.2, 250 MiB 240.7 / 162.8.
+        if ((two || 8ull * N * batch > 40ull << 20) && g < 16) g = 16;
         if (n1 < g) fail(FG_ERR_INTERNAL, "digit split leaves fewer rows than a tile");
         TileGeom t{};
         t.t0n = (uint32_t)(n1 / g);
@@ -576,9 +587,8 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         // 45.9 / 42.0, 49.3 / 46.0, 53.6 / 49.6, 2^23 67.1 / 62.5; 96 MiB 68.0
         // / 67.4, 75.8 / 71.4, 79.6 / 75.7; 128 MiB 2^16 86.5 / 88.8, 2^24
         // 128.2 / 131.2.  The 8-row last pass of 512 points stores through
-        // the caches too: 2^17 32 MiB 28.1 / 27.7, 64 MiB 46.0 / 53.4.
-        const uint64_t bytes = 8ull * N * batch;
-        p->load_cached_ = p->cached_ && p->chunks() == 1 && bytes <= (g < 16 ? 32ull << 20 : 96ull << 20);
+        // the caches too: 2^17 32 MiB 28.1 / 27.7, 40 MiB 32.3 / 34.1.
+        p->load_cached_ = p->cached_ && p->chunks() == 1 && 8ull * N * batch <= (g < 16 ? 32ull << 20 : 96ull << 20);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -858,7 +868,7 @@ void FftPlan::exec(const void* in, void* out, Direction dir, bool normalize, hip
                 uint64_t tiles = s.per_unit * units;
                 uint32_t order = s.tile_order, order_unit = s.order_unit;
                 Dim3 block = s.block;
-                if (const uint32_t w = s.halves && !two ? narrow_width(s.log_l, s.width, tiles, cu_count) : 0) {
+                if (const uint32_t w = s.narrows && !two ? narrow_width(s.log_l, s.width, tiles, cu_count) : 0) {
                     const uint32_t k = s.width / w;  // the geometry steps tiles by the width (add_tile)
                     tiles *= k;
                     g.t0n *= k;

@@ -62,7 +62,7 @@ public:
     // launch i on the stream launch i runs on (chunk_stream()).
     void exec(const void* in, void* out, Direction dir, bool normalize, hipStream_t stream,
               hipEvent_t* events = nullptr) const;
-    // 1, or 2 for multi-pass 1D plans of two or more chunks (unless
+    // 1, or 2 for multi-pass 1D plans whose batch takes the chunk limit (unless
     // set_streams(1) turned the second stream off).
     int streams() const { return (aux_ && use_aux_) ? 2 : 1; }
     // The most streams this plan can run on (2: it has the second stream's
@@ -145,7 +145,7 @@ private:
         uint64_t per_unit = 0;
         uint32_t tile_order = 0;                // tile: TileGeom::remap (FG_TILE_ORDER_*) when the grid
         uint32_t order_unit = 1;                // is a multiple of order_unit, else the natural order
-        bool halves = false;                    // tile: 32 elements per thread, so narrow_width applies
+        bool narrows = false;                   // tile: the kernel has narrow forms (narrow_width)
         uint32_t log_l = 0, width = 0;          // tile: log2 of the pass's length, columns per workgroup
         TileGeom geom{};                        // tile: addressing (flags/scale/remap set at exec)
     };
@@ -253,8 +253,7 @@ bool use_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
 // exchanges in halves (fg_tile_l*_g*_rh): 32-row tiles of 256 points, 16-row
 // tiles of 512 / 1024 points.
 bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
-// Columns per workgroup of a launch of `tiles` tiles of a halves pass (2^log_l
-// points, g columns per tile) in its narrow form; 0: its own tiles.
+// Columns per workgroup of a launch of `tiles` tiles of a pass (2^log_l points, g columns per tile) in its narrow form; 0: its own tiles.
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count);
 // Whether the column FFT of an image with 2^log_rows rows runs as two passes.
 bool split_2d_columns(uint32_t log_rows);

@@ -148,13 +148,6 @@ struct TileStages {
     }
 };
 
-// The 16-element row tiles that load directly: 16 rows or more (128 points).
-// Measured on gfx950, us per execution against the staged form: 2^21 at 16
-// MiB 30.4 -> 29.5, at 112 MiB 114.8 -> 114.1, at 512 MiB 483.8 -> 483.3.
-// The 8-row tile of 512 points lost at 120 MiB (2^17 84.0 -> 84.9).
-template <int G>
-constexpr bool row_tile_direct() { return G >= 16; }
-
 // The same stages on a [row][position] LDS tile.  Stage 0 (radix 16, no
 // twiddles) ran on the positions the thread loaded, t0 + T*m of row c0; its
 // scatter goes to that row, and every gather takes the positions t + T*m of
@@ -222,11 +215,9 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 }
 
 // ROWWISE: input elements of a column are contiguous (ies == 1, rows of a
-// matrix).  Row tiles that row_tile_direct names load a row's Stockham
-// positions t0 + T*m with T consecutive lanes (8*T contiguous bytes per
-// access) and the first exchange turns the tile (RowTileStages); the others
-// load along the rows and turn the tile through LDS first.  Otherwise
-// columns are contiguous (ics == 1) and consecutive lanes load consecutive
+// matrix): T consecutive lanes load a row's Stockham positions t0 + T*m (8*T
+// contiguous bytes per access) and the first exchange turns the tile
+// (RowTileStages).  Otherwise columns are contiguous (ics == 1) and consecutive lanes load consecutive
 // columns.  Output always has ocs == 1.
 // LOAD_CACHED / STORE_CACHED select the pass's cache policy (gload/gstore).
 // CONJ: the body reads the inverse's conjugation flags; forward passes
@@ -235,7 +226,7 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 // 32-bit per-lane byte offset, so each access costs no 64-bit vector
 // arithmetic; a tile's offsets stay below 2^32 bytes (one transform or image
 // spans at most 128 MiB).
-template <int LOGL, int LOGE, int G, bool ROWWISE, bool DIRECT, bool HALVES_TW, bool LOAD_CACHED, bool STORE_CACHED,
+template <int LOGL, int LOGE, int G, bool ROWWISE, bool HALVES_TW, bool LOAD_CACHED, bool STORE_CACHED,
           bool CONJ>
 __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
@@ -250,34 +241,12 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
     char* out_tile = reinterpret_cast<char*>(out + tc.ob);
 
     float2 x[Sh::E];
-    static_assert(ROWWISE || !DIRECT, "DIRECT is a way to load rows");
-    const int c0 = DIRECT ? tid / Sh::T : c, q0 = DIRECT ? tid % Sh::T : q;
-    if constexpr (DIRECT) {
+    const int c0 = ROWWISE ? tid / Sh::T : c, q0 = ROWWISE ? tid % Sh::T : q;
+    if constexpr (ROWWISE) {
         const char* row = in_tile + (uint32_t)((c0 * g.ics + q0) * sizeof(float2));
 #pragma unroll
         for (int m = 0; m < Sh::E; ++m)
             x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(row) + Sh::T * m);
-    } else if constexpr (ROWWISE) {
-        using Lay = TileLayout<LOGL, G>;
-        constexpr int THREADS = G * Sh::T;
-        // Coalesced along each row: linear element li -> (column li / L, position li % L).
-#pragma unroll
-        for (int m = 0; m < Sh::E; ++m) {
-            const int li = tid + THREADS * m;
-            const int cc = li >> LOGL;
-            const int n = li & (Sh::N - 1);
-            const uint32_t off = (uint32_t)((cc * g.ics + n) * sizeof(float2));
-            lds[Lay::at(n, cc)] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(in_tile + off));
-        }
-        __syncthreads();
-        if constexpr (!Lay::PADPOS || Sh::T % 16 == 0) {
-            const float2* base = lds + Lay::at(q, c);
-#pragma unroll
-            for (int m = 0; m < Sh::E; ++m) x[m] = base[m * Lay::template step<Sh::T>()];
-        } else {
-#pragma unroll
-            for (int m = 0; m < Sh::E; ++m) x[m] = lds[Lay::at(q + Sh::T * m, c)];
-        }
     } else {
         const uint32_t lane_off = (uint32_t)((c + (uint64_t)q * g.ies) * sizeof(float2));
         const uint64_t row_step = (uint64_t)Sh::T * g.ies * sizeof(float2);
@@ -291,7 +260,7 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
             for (int m = 0; m < Sh::E; ++m) x[m] = cconj(x[m]);
         }
     }
-    if constexpr (DIRECT) RowTileStages<LOGL, LOGE, G, 0>::run(x, c0, q0, c, q, tw, lds);
+    if constexpr (ROWWISE) RowTileStages<LOGL, LOGE, G, 0>::run(x, c0, q0, c, q, tw, lds);
     else TileStages<LOGL, LOGE, G, 0>::run(x, q, c, tw, lds);
 
     if (g.log_m != 0) {
@@ -541,9 +510,9 @@ __device__ __forceinline__ void fft_tile_narrow(const float2* __restrict__ in, f
                                                 const TileGeom& g, float2* __restrict__ lds) {
     constexpr bool STORE_CACHED = !(STREAM_OUT && ROWWISE && W >= 16);
     if (g.flags & FG_PASS_CONJ)
-        fft_tile_body<LOGL, 4, W, ROWWISE, ROWWISE, true, true, STORE_CACHED, true>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, true>(in, out, tw, big, g, lds);
     else
-        fft_tile_body<LOGL, 4, W, ROWWISE, ROWWISE, true, true, STORE_CACHED, false>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, false>(in, out, tw, big, g, lds);
 }
 
 // The widths a halves pass can be narrowed to: below its own, at least one
@@ -603,12 +572,15 @@ template <int LOGL, int LOGE, int G, bool ROWWISE, bool LOAD_CACHED, bool STORE_
 __device__ __forceinline__ void fft_tile_pass(const float2* __restrict__ in, float2* __restrict__ out,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g) {
-    constexpr bool DIRECT = ROWWISE && row_tile_direct<G>();
-    __shared__ float2 lds[DIRECT ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
+    __shared__ float2 lds[ROWWISE ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
+    if constexpr (ROWWISE && G == 8) {
+        if (g.flags >> FG_PASS_WIDTH_SHIFT == 4)
+            return fft_tile_narrow<LOGL, 4, ROWWISE, false>(in, out, tw, big, g, lds);
+    }
     if (g.flags & FG_PASS_CONJ)
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, DIRECT, false, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
     else
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, DIRECT, false, LOAD_CACHED, STORE_CACHED, false>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, false>(in, out, tw, big, g, lds);
 }
 
 }  // namespace fg

@@ -209,9 +209,9 @@ FG_API int fg_graph_destroy(fg_graph_t graph);
  * over one chunk (whole transforms or images) before the next, keeping the
  * chunk's intermediate array cached (in the 256 MB Infinity Cache) instead of
  * moving it through HBM.  `bytes` bounds the chunks in flight at once: plans
- * that run two chunks at a time (fg_fft_plan_streams) take chunks of at most
- * bytes / 2 when a transform fits that (else one chunk at a time, of at most
- * `bytes`), the others chunks of at most `bytes`.  The limit applies to plans
+ * that run two chunks at a time (fg_fft_plan_streams: multi-pass 1D plans
+ * whose batch takes `bytes` or more and whose transform fits bytes / 2) take
+ * chunks of at most bytes / 2, the others chunks of at most `bytes`.  The limit applies to plans
  * created afterwards, process-wide; 0 disables chunking (one chunk of the
  * whole batch, every pass streaming).  Default: FERRUM_GPU_CHUNK_MIB from the
  * environment when the library loads, else 256 MiB. */

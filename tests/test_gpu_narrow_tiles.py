@@ -32,7 +32,7 @@ def _run(dev, plan, x, direction, normalize, in_place=False):
 # 128; 2^18: 32 / 16; 2^19, 2^20: 64 / 32 and 64 / 64.  2D: C / width tiles.
 SHAPES = [
     (0, 16, (1, 4, 5, 32, 33, 128), 131),
-    (0, 17, (1, 3, 17), 70),
+    (0, 17, (1, 4, 5, 17, 39), 70),
     (0, 18, (1, 2, 3, 9, 17), 34),
     (0, 19, (1, 5), 18),
     (0, 20, (1, 2, 5), 9),

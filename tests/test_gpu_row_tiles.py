@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 TOL = 5e-6
 
 CASES = [(16, 1, None), (17, 1, None), (17, 5, 4 << 20), (18, 1, None), (18, 3, None), (18, 5, 8 << 20), (19, 1, None),
-         (19, 3, 16 << 20), (20, 1, None), (20, 3, 32 << 20), (21, 1, None), (22, 1, None)]
+         (19, 3, 8 << 20), (20, 1, None), (20, 3, 16 << 20), (21, 1, None), (22, 1, None)]
 
 
 @pytest.mark.parametrize("log_n,batch,limit", CASES)
