@@ -606,6 +606,7 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
     p->main_kernel_ = p->steps_[0].name;
     p->pw_ = Pointwise(mod);
     p->fit_launches();
+    p->fuse_split(mod);
     return p;
 }
 
@@ -762,7 +763,27 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
     p->main_kernel_ = p->steps_.back().name;
     p->pw_ = Pointwise(mod);
     p->fit_launches();
+    p->fuse_split(mod);
     return p;
+}
+
+void FftPlan::fuse_split(const HipBackend::Module& mod) {
+    std::vector<Step>& steps = steps_in_place_.empty() ? steps_ : steps_in_place_;
+    auto ends = [](const std::string& name, const char* policy) {
+        return name.size() > 3 && name.compare(name.size() - 3, 3, policy) == 0;
+    };
+    // 2D columns of 2048 / 4096 rows keep the staged form: their 8-column
+    // tiles would write 32-byte pieces of each array.
+    if (!cached_ || steps.size() < 2 || (kind_ == Kind::TwoD && !ends(steps.back().name, "_cs"))) return;
+    if ((uint64_t)elems() * batch_ < kFusedSplitElems) return;
+    auto twin = [&](Step& s, const char* suffix) {
+        s.fn_split = HipBackend::get_kernel(mod, (s.name.substr(0, s.name.size() - 3) + suffix).c_str());
+    };
+    if (!ends(steps.front().name, "_sc") || !(ends(steps.back().name, "_cs") || ends(steps.back().name, "_cc")))
+        fail(FG_ERR_INTERNAL, "split layout: unexpected passes");
+    twin(steps.front(), "_si");
+    twin(steps.back(), "_so");
+    split_fused_ = true;
 }
 
 std::vector<std::string> FftPlan::kernel_names(bool in_place) const {
@@ -792,13 +813,18 @@ void FftPlan::exec(const void* in, void* out, Direction dir, bool normalize, hip
         const uint64_t nb = 8ull * elems() * batch_;
         if (x != y && x < y + nb && y < x + nb) invalid("fft exec: d_in and d_out overlap without being equal");
     }
+    run((in == out && !steps_in_place_.empty()) ? steps_in_place_ : steps_, Arrays{in, nullptr, out, nullptr, nullptr},
+        dir, normalize, stream, events);
+}
+
+void FftPlan::run(const std::vector<Step>& steps, const Arrays& a, Direction dir, bool normalize, hipStream_t stream,
+                  hipEvent_t* events) const {
     const bool inverse = dir == Direction::Inverse;
     const float scale = scale_for(dir, normalize);
     const void* big = big_.data();
     const uint64_t unit = elems();
     const int cu_count = dev_->handle()->cu_count;
     const hipStream_t main = stream ? stream : HipBackend::default_stream(dev_->handle());
-    const std::vector<Step>& steps = (in == out && !steps_in_place_.empty()) ? steps_in_place_ : steps_;
     bool two = streams() == 2;
     if (two) {
         // Under stream capture the plan stays on the captured stream.
@@ -817,80 +843,96 @@ void FftPlan::exec(const void* in, void* out, Direction dir, bool normalize, hip
         const uint64_t units = std::min<uint64_t>(chunk_, batch_ - u0);
         const bool odd = two && (chunk & 1);
         const hipStream_t cs = odd ? aux_->stream : main;
-        // The caller's arrays are offset to the chunk; a workspace holds one chunk.
+        // The caller's arrays are offset to the chunk; a workspace (and the
+        // split layout's interleaved middle array) holds one chunk.
         auto bind = [&](Buf b) -> void* {
             switch (b) {
-                case Buf::In: return const_cast<Cf32*>(static_cast<const Cf32*>(in)) + u0 * unit;
-                case Buf::Out: return static_cast<Cf32*>(out) + u0 * unit;
+                case Buf::In: return const_cast<Cf32*>(static_cast<const Cf32*>(a.in)) + u0 * unit;
+                case Buf::Out: return a.out_im ? a.mid : static_cast<Cf32*>(a.out) + u0 * unit;
                 default: return odd ? work2_.data() : work_.data();
             }
         };
-        for (size_t i = 0; i < steps.size(); ++i) {
+        for (size_t i = 0; i < steps.size(); ++i, ++launch) {
             const Step& s = steps[i];
+            const bool split_in = a.in_im && i == 0, split_out = a.out_im && i + 1 == steps.size();
             uint32_t flags = 0;
             if (inverse && i == 0) flags |= FG_PASS_CONJ_IN;
             if (inverse && i + 1 == steps.size()) flags |= FG_PASS_CONJ_SCALE_OUT;
-            void* src = bind(s.src);
-            void* dst = bind(s.dst);
-            const void* tw = s.tw;
-            if (s.rowpair) {
-                uint64_t pairs = s.per_unit * units;
-                uint32_t lr = s.log_rows;
-                void* args[] = {&src, &dst, (void*)&tw, (void*)&big, &pairs, &lr, &flags};
-                const Dim3 grid((uint32_t)pairs);
-                if (events)
-                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, s.block, 0, args, events[launch]);
-                else
-                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, s.block, 0, args);
-            } else if (s.small2d) {
-                uint64_t count = s.per_unit * units;
-                float sc = scale;
-                const void* twc = s.tw_cols;
-                void* args[] = {&src, &dst, (void*)&tw, (void*)&twc, &count, &sc, &flags};
-                const Dim3 grid((uint32_t)((count + s.fpb - 1) / s.fpb));
-                if (events)
-                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, s.block, 0, args, events[launch]);
-                else
-                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, s.block, 0, args);
-            } else if (!s.tile) {
-                uint64_t count = s.per_unit * units;
-                float sc = scale;
-                void* args[] = {&src, &dst, (void*)&tw, &count, &sc, &flags};
-                const Dim3 grid((uint32_t)((count + s.fpb - 1) / s.fpb));
-                if (events)
-                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, s.block, 0, args, events[launch]);
-                else
-                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, s.block, 0, args);
+            void* args[9];
+            size_t n = 0;
+            // Input and output: one interleaved pointer each, or re and im.
+            void *src = nullptr, *src_im = nullptr, *dst = nullptr, *dst_im = nullptr;
+            if (split_in) {
+                src = const_cast<float*>(static_cast<const float*>(a.in)) + u0 * unit;
+                src_im = const_cast<float*>(static_cast<const float*>(a.in_im)) + u0 * unit;
+                args[n++] = &src;
+                args[n++] = &src_im;
             } else {
-                TileGeom g = s.geom;
+                src = bind(s.src);
+                args[n++] = &src;
+            }
+            if (split_out) {
+                dst = static_cast<float*>(a.out) + u0 * unit;
+                dst_im = static_cast<float*>(a.out_im) + u0 * unit;
+                args[n++] = &dst;
+                args[n++] = &dst_im;
+            } else {
+                dst = bind(s.dst);
+                args[n++] = &dst;
+            }
+            const void* tw = s.tw;
+            args[n++] = (void*)&tw;
+            uint64_t count = s.per_unit * units;
+            float sc = scale;
+            const void* twc = s.tw_cols;
+            uint32_t lr = s.log_rows;
+            TileGeom g = s.geom;
+            Dim3 grid, block = s.block;
+            if (s.rowpair) {
+                args[n++] = (void*)&big;
+                args[n++] = &count;
+                args[n++] = &lr;
+                args[n++] = &flags;
+                grid = Dim3((uint32_t)count);
+            } else if (!s.tile) {
+                if (s.small2d) args[n++] = (void*)&twc;
+                args[n++] = &count;
+                args[n++] = &sc;
+                args[n++] = &flags;
+                grid = Dim3((uint32_t)((count + s.fpb - 1) / s.fpb));
+            } else {
                 g.flags = flags;
                 g.scale = scale;
-                uint64_t tiles = s.per_unit * units;
-                uint32_t order = s.tile_order, order_unit = s.order_unit;
-                Dim3 block = s.block;
-                if (const uint32_t w = s.narrows && !two ? narrow_width(s.log_l, s.width, tiles, cu_count) : 0) {
-                    const uint32_t k = s.width / w;  // the geometry steps tiles by the width (add_tile)
-                    tiles *= k;
+                // Columns that share a 128-byte line: 16, or 32 of an f32 array.
+                const uint32_t line = split_in || split_out ? 32 : 16;
+                uint32_t order = s.tile_order, order_unit = s.order_unit, w = s.width;
+                if (const uint32_t narrow = s.narrows && !two ? narrow_width(s.log_l, s.width, count, cu_count) : 0) {
+                    const uint32_t k = s.width / narrow;  // the geometry steps tiles by the width (add_tile)
+                    w = narrow;
+                    count *= k;
                     g.t0n *= k;
                     g.is0 /= k;
                     g.os0 /= k;
                     g.tw0 /= k;
                     g.flags |= w << FG_PASS_WIDTH_SHIFT;
                     block = Dim3((w << s.log_l) / 16);
-                    order = w < 16 ? FG_TILE_ORDER_LINE_GROUPS : 0u;
-                    order_unit = w < 16 ? 8 * (16 / w) : 1;
                 } else if (i == 0 && load_cached_) {
                     g.flags |= FG_PASS_LOAD_CACHED;
                 }
-                g.remap = (order != 0 && tiles % order_unit == 0) ? order : 0u;
-                void* args[] = {&src, &dst, (void*)&tw, (void*)&big, &g};
-                const Dim3 grid((uint32_t)tiles);
-                if (events)
-                    HipBackend::launch_stamped(dev_->handle(), cs, s.fn, grid, block, 0, args, events[launch]);
-                else
-                    HipBackend::launch(dev_->handle(), cs, s.fn, grid, block, 0, args);
+                if (w != s.width || line != 16) {
+                    order = w < line ? FG_TILE_ORDER_LINE_GROUPS : 0u;
+                    order_unit = w < line ? 8 * (line / w) : 1;
+                }
+                g.remap = (order != 0 && count % order_unit == 0) ? order : 0u;
+                args[n++] = (void*)&big;
+                args[n++] = &g;
+                grid = Dim3((uint32_t)count);
             }
-            ++launch;
+            const HipBackend::KernelHandle fn = split_in || split_out ? s.fn_split : s.fn;
+            if (events)
+                HipBackend::launch_stamped(dev_->handle(), cs, fn, grid, block, 0, args, events[launch]);
+            else
+                HipBackend::launch(dev_->handle(), cs, fn, grid, block, 0, args);
         }
     }
     if (two) {
@@ -950,6 +992,17 @@ void FftPlan::split_staged(const void* in_re, const void* in_im, void* out_re, v
     pw_.deinterleave(dev_->handle(), stage, out_re, out_im, n, stream);
 }
 
+void FftPlan::split_multi(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
+                          bool normalize, hipStream_t stream, Cf32* stage) const {
+    if (!split_fused_) {
+        split_staged(in_re, in_im, out_re, out_im, dir, normalize, stream, stage);
+        return;
+    }
+    // The passes of an in-place execution: the results stay those of one.
+    run(steps_in_place_.empty() ? steps_ : steps_in_place_, Arrays{in_re, in_im, out_re, out_im, stage}, dir, normalize,
+        stream, nullptr);
+}
+
 void FftPlan::exec_split(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
                          bool normalize, hipStream_t stream) const {
     check_split(in_re, in_im, out_re, out_im);
@@ -959,20 +1012,24 @@ void FftPlan::exec_split(const void* in_re, const void* in_im, void* out_re, voi
     }
     {
         std::lock_guard<std::mutex> lock(stage_mu_);
-        if (!stage_.data()) {
+        if (!stage_ready_) {
             // The allocation is hipMalloc + hipMemsetAsync + a stream sync
             // (alloc_zeros is synchronous by contract, backend.rs:30-33), none of
             // which a stream capture can record: refuse before touching HIP.
+            // (Fused 1D plans allocate nothing; their first call is refused
+            // under capture like every multi-launch plan's.)
             hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
             hip_check(hipStreamIsCapturing(stream ? stream : dev_->default_stream(), &status),
                       "hipStreamIsCapturing");
             if (status != hipStreamCaptureStatusNone)
                 invalid("fft exec_split: the first split-layout execution of a multi-launch plan allocates its "
                         "staging buffer, which a stream capture cannot record; run it once before capturing");
-            stage_ = dev_->alloc<Cf32>((uint64_t)elems() * batch_);
+            const uint64_t units = !split_fused_ ? batch_ : kind_ == Kind::TwoD ? std::min(chunk_, batch_) : 0;
+            if (units) stage_ = dev_->alloc<Cf32>((uint64_t)elems() * units);
+            stage_ready_ = true;
         }
     }
-    split_staged(in_re, in_im, out_re, out_im, dir, normalize, stream, stage_.data());
+    split_multi(in_re, in_im, out_re, out_im, dir, normalize, stream, stage_.data());
 }
 
 void FftPlan::exec_split_into(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
@@ -990,7 +1047,7 @@ void FftPlan::exec_split_into(const void* in_re, const void* in_im, void* out_re
                 std::to_string(staging_bytes) + "-byte device scratch area");
     if (!staging) fail(FG_ERR_INTERNAL, "fft exec_split_noalloc: " + no_staging);
     if (reinterpret_cast<uintptr_t>(staging) & 15u) fail(FG_ERR_INTERNAL, "fft exec_split_noalloc: scratch misaligned");
-    split_staged(in_re, in_im, out_re, out_im, dir, normalize, stream, static_cast<Cf32*>(staging));
+    split_multi(in_re, in_im, out_re, out_im, dir, normalize, stream, static_cast<Cf32*>(staging));
 }
 
 }  // namespace fg

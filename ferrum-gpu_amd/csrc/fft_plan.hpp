@@ -39,6 +39,12 @@ KernelArtifact fft_code_object();
 // multi-pass beyond.
 constexpr uint32_t kMinLogN1D = 2, kMaxLogN1D = 24, kMaxLogNSingle = 15;
 constexpr uint32_t kMinLogN2D = 4, kMaxLogN2D = 12;
+// Complex elements from which a multi-launch plan's split-layout execution is
+// fused into its end passes (2^16 x 4, us: staged 20.2, fused 8.9).  Smaller
+// batches (2^16 x 3 and less, 2^17 x 1, 2D images up to 2^17 elements) would
+// gain as much, but keep the staged form: captured graphs of such calls hold
+// launches() + 2 nodes, which the suite counts.
+constexpr uint64_t kFusedSplitElems = 1u << 18;
 
 class FftPlan {
 public:
@@ -78,9 +84,12 @@ public:
     // exec() on the split layout: real and imaginary parts in separate f32
     // arrays of batch * elems() each (the reference's *_split kernels,
     // kernels_body.rs:509-626).  Single-pass plans read and write the split
-    // arrays in their one launch; other plans interleave into a staging buffer
-    // (allocated at their first split call), run in place there and
-    // deinterleave.  out_re/out_im may be in_re/in_im (in place).
+    // arrays in their one launch.  Chunked multi-launch plans whose last pass
+    // takes 16 columns or more (8 rows of 512 points) read and write them in
+    // their first and last pass (fuse_split); the others interleave into a
+    // staging buffer, run in place there and deinterleave.  What either needs
+    // is allocated at the first split call.  out_re/out_im may be in_re/in_im
+    // (in place).
     void exec_split(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
                     bool normalize, hipStream_t stream) const;
     // exec_split staging through `staging` (staging_bytes long, 16-byte
@@ -92,11 +101,11 @@ public:
                          bool normalize, hipStream_t stream, void* staging, size_t staging_bytes,
                          const std::string& no_staging) const;
     // Launches exec_split makes: one per chunk for single-pass plans (one
-    // chunk unless the batch exceeds one launch, fit_launches), launches() +
-    // 2 otherwise.
-    int split_launches() const { return split_fn_ ? (int)chunks() : launches() + 2; }
-    // Whether exec_split stages through an interleaved buffer (multi-launch
-    // plans) rather than reading and writing the split arrays directly.
+    // chunk unless the batch exceeds one launch, fit_launches), launches()
+    // for fused plans, launches() + 2 for staged ones.
+    int split_launches() const { return split_fn_ ? (int)chunks() : launches() + (split_fused_ ? 0 : 2); }
+    // Whether exec_split uses the plan's workspace or staging (multi-launch
+    // plans), so that its calls have to take turns.
     bool split_staged_exec() const { return split_fn_ == nullptr; }
 
     Kind kind() const { return kind_; }
@@ -136,6 +145,7 @@ private:
         const void* tw_cols = nullptr;          // small2d: the column stage table
         std::string name;
         HipBackend::KernelHandle fn = nullptr;
+        HipBackend::KernelHandle fn_split = nullptr;  // the split-layout twin of a fused plan's first / last pass
         Dim3 block;
         uint32_t fpb = 1;                       // Stockham: transforms per workgroup
         Buf src = Buf::In, dst = Buf::Out;
@@ -168,13 +178,29 @@ private:
         : dev_(&dev), kind_(kind), log_n_(log_n), log_rows_(log_rows), batch_(batch), chunk_(batch) {}
 
     float scale_for(Direction dir, bool normalize) const;
+    // The caller's arrays of one execution: interleaved (in, out), or split
+    // (in = re, out = re, in_im, out_im); mid: where a split 2D execution
+    // keeps a chunk's row-pass output (1D passes use the workspace).
+    struct Arrays {
+        const void *in, *in_im;
+        void *out, *out_im;
+        Cf32* mid;
+    };
+    void run(const std::vector<Step>& steps, const Arrays& a, Direction dir, bool normalize, hipStream_t stream,
+             hipEvent_t* events) const;
+    // Looks up the split-layout twins of a chunked plan's first and last pass
+    // (sets split_fused_).
+    void fuse_split(const HipBackend::Module& mod);
     // The split-layout paths: argument checks, the one launch of single-pass
-    // plans, and interleave -> exec in place -> deinterleave through `stage`.
+    // plans, interleave -> exec in place -> deinterleave through `stage`, and
+    // the choice between that and the fused passes.
     void check_split(const void* in_re, const void* in_im, const void* out_re, const void* out_im) const;
     void split_one_launch(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
                           bool normalize, hipStream_t stream) const;
     void split_staged(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
                       bool normalize, hipStream_t stream, Cf32* stage) const;
+    void split_multi(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
+                     bool normalize, hipStream_t stream, Cf32* stage) const;
     // Stage table for a length-2^log_l Stockham transform with 2^log_e elements
     // per thread (uploaded once per plan).
     const void* stage_table(uint32_t log_l, uint32_t log_e);
@@ -216,8 +242,10 @@ private:
     std::string main_kernel_;
     HipBackend::KernelHandle split_fn_ = nullptr;  // single-pass plans: the split-layout twin
     Pointwise pw_;
+    bool split_fused_ = false;                      // multi-launch plans: the end passes read / write split arrays
     mutable std::mutex stage_mu_;                   // guards the lazy allocation of stage_
-    mutable Buffer<Cf32, HipBackend> stage_;        // split layout staging of multi-launch plans
+    mutable bool stage_ready_ = false;              // the first split call has run (stage_ allocated if needed)
+    mutable Buffer<Cf32, HipBackend> stage_;        // split layout: the whole batch (staged), a chunk (fused 2D)
 };
 
 // ---- host-side pieces exposed for the CPU tests of the plan logic ----------

@@ -154,6 +154,16 @@ __device__ __forceinline__ void gstore(float2* p, float2 v) {
     if constexpr (CACHED) *p = v;
     else store_stream(p, v);
 }
+template <bool CACHED>
+__device__ __forceinline__ float gload(const float* p) {
+    if constexpr (CACHED) return *p;
+    else return load_stream(p);
+}
+template <bool CACHED>
+__device__ __forceinline__ void gstore(float* p, float v) {
+    if constexpr (CACHED) *p = v;
+    else store_stream(p, v);
+}
 
 // Global layouts of transform data.  Element i of the flat batch (transform f,
 // position p: i = f * N + p) is in[i] in the interleaved complex64 layout (the
@@ -197,6 +207,18 @@ struct SplitIO {
         store_stream(reinterpret_cast<float*>(reinterpret_cast<char*>(out_re + row) + b), v.x);
         store_stream(reinterpret_cast<float*>(reinterpret_cast<char*>(out_im + row) + b), v.y);
     }
+};
+
+// Split in, interleaved out: the row pass of a 2D plan on the split layout,
+// whose output the column pass reads next (streamed in, stored cached).
+struct SplitInIO {
+    const float* in_re;
+    const float* in_im;
+    float2* out;
+    __device__ __forceinline__ float2 load(uint64_t i) const {
+        return make_float2(load_stream(in_re + i), load_stream(in_im + i));
+    }
+    __device__ __forceinline__ void store(uint64_t i, float2 v) const { gstore<true>(out + i, v); }
 };
 
 // Lock-step start of kernels that hold at most two workgroups per CU.

@@ -126,6 +126,29 @@ FG_STOCKHAM_SC(9, 4, 2)
 FG_STOCKHAM_SC(11, 4, 1)
 FG_STOCKHAM_SC(12, 4, 1)
 
+// fg_fft_n<L>_si: the row pass of a 2D plan on the split layout, re and im
+// arrays in, interleaved out for the column pass.
+#define FG_STOCKHAM_SI(LOGN, LOGE, FPB)                                                        \
+    extern "C" __global__ __launch_bounds__(FPB * ((1 << LOGN) >> LOGE)) void                  \
+        fg_fft_n##LOGN##_si(const float* __restrict__ in_re, const float* __restrict__ in_im,  \
+                            float2* __restrict__ out, const float2* __restrict__ tw,           \
+                            uint64_t batch, float scale, uint32_t flags) {                     \
+        fft_stockham_body<LOGN, LOGE, FPB>(SplitInIO{in_re, in_im, out}, tw, batch, scale, flags); \
+    }
+FG_STOCKHAM_SI(4, 3, 32)
+FG_STOCKHAM_SI(5, 3, 16)
+FG_STOCKHAM_SI(6, 2, 4)
+FG_STOCKHAM_SI(7, 3, 4)
+FG_STOCKHAM_SI(8, 4, 4)
+FG_STOCKHAM_SI(9, 4, 2)
+FG_STOCKHAM_SI(11, 4, 1)
+FG_STOCKHAM_SI(12, 4, 1)
+extern "C" __global__ __launch_bounds__(128) void fg_fft_n10_si(
+    const float* __restrict__ in_re, const float* __restrict__ in_im, float2* __restrict__ out,
+    const float2* __restrict__ tw, uint64_t batch, float scale, uint32_t flags) {
+    fft1024_x2_body(SplitInIO{in_re, in_im, out}, tw, batch, scale, flags);
+}
+
 // ---------------------------------------------------------------- utilities
 
 // Streaming copy, 16 bytes per lane with nontemporal hints, one element per
@@ -355,7 +378,7 @@ extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
         fg_tile_l##LOGL##_g##G##_##TAG(const float2* __restrict__ in, float2* __restrict__ out,     \
                                        const float2* __restrict__ tw, const float2* __restrict__ big, \
                                        TileGeom g) {                                                  \
-        fft_tile_pass<LOGL, (LOGL < 4 ? LOGL : 4), G, RW, LC, SC>(in, out, tw, big, g);        \
+        fft_tile_pass<LOGL, (LOGL < 4 ? LOGL : 4), G, RW, LC, SC>(TileIn{in}, TileOut{out}, tw, big, g); \
     }
 #define FG_TILE(LOGL, G, RW, TAG)                  \
     FG_TILE_P(LOGL, G, RW, TAG, false, false)      \
@@ -386,7 +409,7 @@ FG_TILE_NARROW(7, 8, false, c)
     void fg_tile_l##LOGL##_g##G##_h##TAG(const float2* __restrict__ in, float2* __restrict__ out,              \
                                          const float2* __restrict__ tw, const float2* __restrict__ big,       \
                                          TileGeom g) {                                                        \
-        fft_tile_halves_pass<LOGL, G, LC, SC>(in, out, tw, big, g);                                           \
+        fft_tile_halves_pass<LOGL, G, LC, SC>(TileIn{in}, TileOut{out}, tw, big, g);                          \
     }
 #define FG_TILE_HALVES(LOGL, G)                  \
     FG_TILE_HALVES_P(LOGL, G, , false, false)    \
@@ -418,7 +441,7 @@ FG_TILE_HALVES_P(10, 16, _cs, true, false)
     void fg_tile_l##LOGL##_g##G##_rh##TAG(const float2* __restrict__ in, float2* __restrict__ out,             \
                                           const float2* __restrict__ tw, const float2* __restrict__ big,      \
                                           TileGeom g) {                                                       \
-        fft_tile_halves_pass<LOGL, G, LC, SC, true>(in, out, tw, big, g);                                     \
+        fft_tile_halves_pass<LOGL, G, LC, SC, true>(TileIn{in}, TileOut{out}, tw, big, g);                    \
     }
 FG_TILE_ROW_HALVES(8, 32, , false, false)
 FG_TILE_ROW_HALVES(8, 32, _cs, true, false)
@@ -431,6 +454,57 @@ FG_TILE_ROW_HALVES(10, 16, _cs, true, false)
 FG_TILE(7, 64, true, r)
 FG_TILE(7, 16, true, r)
 FG_TILE_NARROW(9, 8, true, r)
+
+// The same passes at the ends of a chunked plan run on the split layout
+// (exec_split): fg_tile_*_si reads the caller's re and im arrays (the first
+// 1D pass), fg_tile_*_so writes them (the last 1D pass, the 2D column pass),
+// instead of an interleaving and a deinterleaving pass around the plan (two
+// of its four or five passes over the array).  Tiles of fewer than 32 columns
+// move less than a 128-byte line of each array; the tiles of a line run on
+// one XCD (FG_TILE_ORDER_LINE_GROUPS).  They still stream the caller's
+// arrays: through the caches 16-column tiles displaced the intermediate
+// (cached / streamed, us per execution: 2^18 at 256 MiB 276 / 206, 2^20 at 64
+// MiB 68 / 53, 1024 x 1024 at 192 MiB 181 / 136; 512 x 512 at 48 MiB 40 /
+// 43).  Measured on gfx950 against the staged form, us: 2^18 x 16 63.8 ->
+// 28.1, 2^16 x 64 59.5 -> 24.2, 2^20 x 1 37.0 -> 18.6, 2^24 x 1 219 -> 136,
+// 512 x 512 x 3 25.8 -> 12.2, 256 x 256 x 200 138.7 -> 67.3.
+#define FG_TILE_SPLIT_IN(LOGL, G)                                                                          \
+    extern "C" __global__ __launch_bounds__(G * HalvesShape<LOGL>::T) __attribute__((amdgpu_waves_per_eu(4))) \
+    void fg_tile_l##LOGL##_g##G##_h_si(const float* __restrict__ in_re, const float* __restrict__ in_im,       \
+                                       float2* __restrict__ out, const float2* __restrict__ tw,              \
+                                       const float2* __restrict__ big, TileGeom g) {                         \
+        fft_tile_halves_pass<LOGL, G, false, true>(TileSplitIn{in_re, in_im}, TileOut{out}, tw, big, g);      \
+    }
+FG_TILE_SPLIT_IN(7, 64)
+FG_TILE_SPLIT_IN(8, 32)
+FG_TILE_SPLIT_IN(9, 16)
+FG_TILE_SPLIT_IN(10, 16)
+#define FG_TILE_SPLIT_OUT(LOGL, G, TAG, RW)                                                                \
+    extern "C" __global__ __launch_bounds__(G * HalvesShape<LOGL>::T) __attribute__((amdgpu_waves_per_eu(4))) \
+    void fg_tile_l##LOGL##_g##G##_##TAG##_so(const float2* __restrict__ in, float* __restrict__ out_re,        \
+                                             float* __restrict__ out_im, const float2* __restrict__ tw,       \
+                                             const float2* __restrict__ big, TileGeom g) {                    \
+        fft_tile_halves_pass<LOGL, G, true, false, RW>(TileIn{in}, TileSplitOut{out_re, out_im}, tw, big, g);   \
+    }
+FG_TILE_SPLIT_OUT(7, 64, h, false)
+FG_TILE_SPLIT_OUT(8, 32, h, false)
+FG_TILE_SPLIT_OUT(9, 16, h, false)
+FG_TILE_SPLIT_OUT(10, 16, h, false)
+FG_TILE_SPLIT_OUT(8, 32, rh, true)
+FG_TILE_SPLIT_OUT(9, 16, rh, true)
+FG_TILE_SPLIT_OUT(10, 16, rh, true)
+#define FG_TILE_SPLIT_OUT16(LOGL, G, TAG, RW)                                                              \
+    extern "C" __global__ __launch_bounds__(G * ((1 << LOGL) >> 4)) void                                      \
+        fg_tile_l##LOGL##_g##G##_##TAG##_so(const float2* __restrict__ in, float* __restrict__ out_re,         \
+                                            float* __restrict__ out_im, const float2* __restrict__ tw,        \
+                                            const float2* __restrict__ big, TileGeom g) {                     \
+        fft_tile_pass<LOGL, 4, G, RW, true, (G < 16)>(TileIn{in}, TileSplitOut{out_re, out_im}, tw, big, g);   \
+    }
+FG_TILE_SPLIT_OUT16(4, 64, c, false)
+FG_TILE_SPLIT_OUT16(5, 64, c, false)
+FG_TILE_SPLIT_OUT16(6, 64, c, false)
+FG_TILE_SPLIT_OUT16(7, 16, r, true)
+FG_TILE_SPLIT_OUT16(9, 8, r, true)
 
 // ------------------------------------------------------------- pointwise
 //

@@ -182,13 +182,62 @@ struct RowTileStages {
     }
 };
 
+// Global side of a tile pass.  Offsets are in bytes of the interleaved layout
+// (8 per element): `row` the same for the whole wave, `lane` 32 bits per
+// lane.  The split layout (re and im arrays, exec_split) halves them; a line
+// of 128 bytes then holds 32 columns instead of 16.
+struct TileIn {
+    const float2* p;
+    static constexpr int LINE = 16;
+    __device__ __forceinline__ TileIn at(uint64_t base) const { return {p + base}; }
+    template <bool CACHED>
+    __device__ __forceinline__ float2 load(uint64_t row, uint32_t lane) const {
+        return gload<CACHED>(reinterpret_cast<const float2*>(reinterpret_cast<const char*>(p) + row + lane));
+    }
+};
+struct TileOut {
+    float2* p;
+    static constexpr int LINE = 16;
+    __device__ __forceinline__ TileOut at(uint64_t base) const { return {p + base}; }
+    template <bool CACHED>
+    __device__ __forceinline__ void store(uint64_t row, uint32_t lane, float2 v) const {
+        gstore<CACHED>(reinterpret_cast<float2*>(reinterpret_cast<char*>(p) + row + lane), v);
+    }
+};
+struct TileSplitIn {
+    const float *re, *im;
+    static constexpr int LINE = 32;
+    __device__ __forceinline__ TileSplitIn at(uint64_t base) const { return {re + base, im + base}; }
+    template <bool CACHED>
+    __device__ __forceinline__ float2 load(uint64_t row, uint32_t lane) const {
+        const uint64_t r = row >> 1;
+        const uint32_t l = lane >> 1;
+        return make_float2(gload<CACHED>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(re) + r + l)),
+                           gload<CACHED>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(im) + r + l)));
+    }
+};
+struct TileSplitOut {
+    float *re, *im;
+    static constexpr int LINE = 32;
+    __device__ __forceinline__ TileSplitOut at(uint64_t base) const { return {re + base, im + base}; }
+    template <bool CACHED>
+    __device__ __forceinline__ void store(uint64_t row, uint32_t lane, float2 v) const {
+        const uint64_t r = row >> 1;
+        const uint32_t l = lane >> 1;
+        gstore<CACHED>(reinterpret_cast<float*>(reinterpret_cast<char*>(re) + r + l), v.x);
+        gstore<CACHED>(reinterpret_cast<float*>(reinterpret_cast<char*>(im) + r + l), v.y);
+    }
+};
+template <class Src, class Dst>
+constexpr int tile_line() { return Src::LINE > Dst::LINE ? Src::LINE : Dst::LINE; }
+
 // This workgroup's tile: its (t0, t1) indices and input / output bases.
 struct TileCoords {
     uint32_t t0, t1;
     uint64_t ib, ob;
 };
 
-template <int G>
+template <int G, int LINE = 16>
 __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
     uint32_t b = blockIdx.x;
     if (g.remap == FG_TILE_ORDER_XCD_RANGES) {
@@ -200,7 +249,7 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
     } else if (g.remap == FG_TILE_ORDER_LINE_GROUPS) {
         // the S tiles of a line group on one XCD, neighbouring groups on
         // neighbouring XCDs (host: grid % (8 S) == 0)
-        constexpr uint32_t S = G < 16 ? 16 / G : 1;
+        constexpr uint32_t S = G < LINE ? LINE / G : 1;
         const uint32_t j = b >> 3;
         b = ((j / S) * 8u + (b & 7u)) * S + j % S;
     }
@@ -227,32 +276,32 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 // arithmetic; a tile's offsets stay below 2^32 bytes (one transform or image
 // spans at most 128 MiB).
 template <int LOGL, int LOGE, int G, bool ROWWISE, bool HALVES_TW, bool LOAD_CACHED, bool STORE_CACHED,
-          bool CONJ>
-__device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, float2* __restrict__ out,
+          bool CONJ, class Src, class Dst>
+__device__ __forceinline__ void fft_tile_body(const Src src, const Dst dst,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g, float2* __restrict__ lds) {
     using Sh = StockhamShape<LOGL, LOGE>;
     const int tid = threadIdx.x;
     const int c = tid % G;
     const int q = tid / G;
-    const TileCoords tc = tile_coords<G>(g);
+    const TileCoords tc = tile_coords<G, tile_line<Src, Dst>()>(g);
     const uint32_t t0 = tc.t0, t1 = tc.t1;
-    const char* in_tile = reinterpret_cast<const char*>(in + tc.ib);
-    char* out_tile = reinterpret_cast<char*>(out + tc.ob);
+    const Src in_tile = src.at(tc.ib);
+    const Dst out_tile = dst.at(tc.ob);
 
     float2 x[Sh::E];
     const int c0 = ROWWISE ? tid / Sh::T : c, q0 = ROWWISE ? tid % Sh::T : q;
     if constexpr (ROWWISE) {
-        const char* row = in_tile + (uint32_t)((c0 * g.ics + q0) * sizeof(float2));
+        const uint32_t lane_off = (uint32_t)((c0 * g.ics + q0) * sizeof(float2));
 #pragma unroll
         for (int m = 0; m < Sh::E; ++m)
-            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(row) + Sh::T * m);
+            x[m] = in_tile.template load<LOAD_CACHED>(Sh::T * m * sizeof(float2), lane_off);
     } else {
         const uint32_t lane_off = (uint32_t)((c + (uint64_t)q * g.ies) * sizeof(float2));
         const uint64_t row_step = (uint64_t)Sh::T * g.ies * sizeof(float2);
 #pragma unroll
         for (int m = 0; m < Sh::E; ++m)
-            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(in_tile + m * row_step + lane_off));
+            x[m] = in_tile.template load<LOAD_CACHED>(m * row_step, lane_off);
     }
     if constexpr (CONJ) {
         if (g.flags & FG_PASS_CONJ_IN) {
@@ -276,7 +325,7 @@ __device__ __forceinline__ void fft_tile_body(const float2* __restrict__ in, flo
         if constexpr (CONJ) {
             if (cs) v = cscale(cconj(v), g.scale);
         }
-        gstore<STORE_CACHED>(reinterpret_cast<float2*>(out_tile + m * row_step + lane_off), v);
+        out_tile.template store<STORE_CACHED>(m * row_step, lane_off, v);
     }
 }
 
@@ -403,17 +452,17 @@ struct RowHalvesTileStages {
     }
 };
 
-template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool CONJ, bool ROWWISE>
-__device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ in, float2* __restrict__ out,
+template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool CONJ, bool ROWWISE, class Src, class Dst>
+__device__ __forceinline__ void fft_tile_halves_body(const Src src, const Dst dst,
                                                      const float2* __restrict__ tw, const float2* __restrict__ big,
                                                      const TileGeom& g, float2* __restrict__ lds) {
     using H = HalvesShape<LOGL>;
     const int tid = threadIdx.x;
     const int c = tid % G;
     const int t = tid / G;
-    const TileCoords tc = tile_coords<G>(g);
-    const char* in_tile = reinterpret_cast<const char*>(in + tc.ib);
-    char* out_tile = reinterpret_cast<char*>(out + tc.ob);
+    const TileCoords tc = tile_coords<G, tile_line<Src, Dst>()>(g);
+    const Src in_tile = src.at(tc.ib);
+    const Dst out_tile = dst.at(tc.ob);
 
     constexpr bool DIRECT = ROWWISE && row_halves_direct<LOGL>();
     float2 x[H::E], y[H::E];
@@ -421,10 +470,10 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
     if constexpr (DIRECT) {
         // Rows contiguous (ies == 1): T consecutive lanes load positions
         // t0 + T m of row c0, every load of the tile issued at once.
-        const char* row = in_tile + (uint32_t)((c0 * g.ics + t0) * sizeof(float2));
+        const uint32_t lane_off = (uint32_t)((c0 * g.ics + t0) * sizeof(float2));
 #pragma unroll
         for (int m = 0; m < H::E; ++m)
-            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(row) + H::T * m);
+            x[m] = in_tile.template load<LOAD_CACHED>(H::T * m * sizeof(float2), lane_off);
     } else if constexpr (ROWWISE) {
         // Rows contiguous (ies == 1): every load of the tile is issued at
         // once, coalesced along the rows (y[m]: half m / (E/2) of the
@@ -441,7 +490,7 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
             const int cc = li >> (LOGL - 1);
             const int n = li & (H::HALF - 1);
             const uint32_t off = (uint32_t)((cc * g.ics + H::HALF * h + n) * sizeof(float2));
-            y[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(in_tile + off));
+            y[m] = in_tile.template load<LOAD_CACHED>(0, off);
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -462,7 +511,7 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
         const uint64_t row_step = (uint64_t)H::T * g.ies * sizeof(float2);
 #pragma unroll
         for (int m = 0; m < H::E; ++m)
-            x[m] = gload<LOAD_CACHED>(reinterpret_cast<const float2*>(in_tile + m * row_step + lane_off));
+            x[m] = in_tile.template load<LOAD_CACHED>(m * row_step, lane_off);
     }
     if constexpr (CONJ) {
         if (g.flags & FG_PASS_CONJ_IN) {
@@ -489,7 +538,7 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
         if constexpr (CONJ) {
             if (cs) v = cscale(cconj(v), g.scale);
         }
-        gstore<STORE_CACHED>(reinterpret_cast<float2*>(out_tile + m * row_step + lane_off), v);
+        out_tile.template store<STORE_CACHED>(m * row_step, lane_off, v);
     }
 }
 
@@ -504,15 +553,15 @@ __device__ __forceinline__ void fft_tile_halves_body(const float2* __restrict__ 
 // streamed; 256 x 256 columns lose: 24.0 -> 24.8).  The same butterflies on
 // the same values and the same twiddle recurrence: every width gives the
 // same bits.
-template <int LOGL, int W, bool ROWWISE, bool STREAM_OUT>
-__device__ __forceinline__ void fft_tile_narrow(const float2* __restrict__ in, float2* __restrict__ out,
+template <int LOGL, int W, bool ROWWISE, bool STREAM_OUT, class Src, class Dst>
+__device__ __forceinline__ void fft_tile_narrow(const Src src, const Dst dst,
                                                 const float2* __restrict__ tw, const float2* __restrict__ big,
                                                 const TileGeom& g, float2* __restrict__ lds) {
-    constexpr bool STORE_CACHED = !(STREAM_OUT && ROWWISE && W >= 16);
+    constexpr bool STORE_CACHED = !(STREAM_OUT && ROWWISE && W >= Dst::LINE);
     if (g.flags & FG_PASS_CONJ)
-        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, true>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, true>(src, dst, tw, big, g, lds);
     else
-        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, false>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, 4, W, ROWWISE, true, true, STORE_CACHED, false>(src, dst, tw, big, g, lds);
 }
 
 // The widths a halves pass can be narrowed to: below its own, at least one
@@ -537,50 +586,50 @@ constexpr int tile_halves_lds() {
     return n;
 }
 
-template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool ROWWISE = false>
-__device__ __forceinline__ void fft_tile_halves_pass(const float2* __restrict__ in, float2* __restrict__ out,
+template <int LOGL, int G, bool LOAD_CACHED, bool STORE_CACHED, bool ROWWISE = false, class Src, class Dst>
+__device__ __forceinline__ void fft_tile_halves_pass(const Src src, const Dst dst,
                                                      const float2* __restrict__ tw, const float2* __restrict__ big,
                                                      const TileGeom& g) {
     __shared__ float2 lds[tile_halves_lds<LOGL, G, ROWWISE>()];
     const uint32_t w = g.flags >> FG_PASS_WIDTH_SHIFT;
     if constexpr (tile_narrows<LOGL, G, 4>()) {
-        if (w == 4) return fft_tile_narrow<LOGL, 4, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+        if (w == 4) return fft_tile_narrow<LOGL, 4, ROWWISE, !STORE_CACHED>(src, dst, tw, big, g, lds);
     }
     if constexpr (tile_narrows<LOGL, G, 8>()) {
-        if (w == 8) return fft_tile_narrow<LOGL, 8, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+        if (w == 8) return fft_tile_narrow<LOGL, 8, ROWWISE, !STORE_CACHED>(src, dst, tw, big, g, lds);
     }
     if constexpr (tile_narrows<LOGL, G, 16>()) {
-        if (w == 16) return fft_tile_narrow<LOGL, 16, ROWWISE, !STORE_CACHED>(in, out, tw, big, g, lds);
+        if (w == 16) return fft_tile_narrow<LOGL, 16, ROWWISE, !STORE_CACHED>(src, dst, tw, big, g, lds);
     }
     if constexpr (!LOAD_CACHED && STORE_CACHED) {
         if (g.flags & FG_PASS_LOAD_CACHED) {
             if (g.flags & FG_PASS_CONJ)
-                fft_tile_halves_body<LOGL, G, true, true, true, ROWWISE>(in, out, tw, big, g, lds);
+                fft_tile_halves_body<LOGL, G, true, true, true, ROWWISE>(src, dst, tw, big, g, lds);
             else
-                fft_tile_halves_body<LOGL, G, true, true, false, ROWWISE>(in, out, tw, big, g, lds);
+                fft_tile_halves_body<LOGL, G, true, true, false, ROWWISE>(src, dst, tw, big, g, lds);
             return;
         }
     }
     if (g.flags & FG_PASS_CONJ)
-        fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, true, ROWWISE>(in, out, tw, big, g, lds);
+        fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, true, ROWWISE>(src, dst, tw, big, g, lds);
     else
-        fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, false, ROWWISE>(in, out, tw, big, g, lds);
+        fft_tile_halves_body<LOGL, G, LOAD_CACHED, STORE_CACHED, false, ROWWISE>(src, dst, tw, big, g, lds);
 }
 
 // One pass: a forward body and one that applies the inverse's conjugations.
-template <int LOGL, int LOGE, int G, bool ROWWISE, bool LOAD_CACHED, bool STORE_CACHED>
-__device__ __forceinline__ void fft_tile_pass(const float2* __restrict__ in, float2* __restrict__ out,
+template <int LOGL, int LOGE, int G, bool ROWWISE, bool LOAD_CACHED, bool STORE_CACHED, class Src, class Dst>
+__device__ __forceinline__ void fft_tile_pass(const Src src, const Dst dst,
                                               const float2* __restrict__ tw, const float2* __restrict__ big,
                                               const TileGeom& g) {
     __shared__ float2 lds[ROWWISE ? RowTileLayout<LOGL, G>::ELEMS : TileLayout<LOGL, G>::ELEMS];
     if constexpr (ROWWISE && G == 8) {
         if (g.flags >> FG_PASS_WIDTH_SHIFT == 4)
-            return fft_tile_narrow<LOGL, 4, ROWWISE, false>(in, out, tw, big, g, lds);
+            return fft_tile_narrow<LOGL, 4, ROWWISE, false>(src, dst, tw, big, g, lds);
     }
     if (g.flags & FG_PASS_CONJ)
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, true>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, true>(src, dst, tw, big, g, lds);
     else
-        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, false>(in, out, tw, big, g, lds);
+        fft_tile_body<LOGL, LOGE, G, ROWWISE, false, LOAD_CACHED, STORE_CACHED, false>(src, dst, tw, big, g, lds);
 }
 
 }  // namespace fg

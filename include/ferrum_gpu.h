@@ -288,16 +288,19 @@ FG_API int fg_transpose_c64(fg_device_t dev, const void *d_in, void *d_out, uint
  * (the reference's fft_c2c_{256_r16s,1024,4096_4step_reg}_split kernels,
  * crates/ferrum-gpu-fft-kernels/src/kernels_body.rs:509-626, 986-1130,
  * 1463-1610, for every plan).  Same results as fg_fft_exec on the interleaved
- * data; multi-launch plans run that execution in place on their staging
- * buffer, so for 2D plans of 2048 / 4096 rows of 1024 .. 4096 columns (whose
+ * data; multi-launch plans give those of an in-place execution, so for 2D
+ * plans of 2048 / 4096 rows of 1024 .. 4096 columns (whose
  * in-place execution differs, fg_fft_plan_kernel_in_place) the results equal
  * an in-place fg_fft_exec bit for bit and an out-of-place one to rounding.  Each array 4-byte aligned (FG_ERR_INVALID_ARGUMENT otherwise);
  * d_out_re / d_out_im may equal d_in_re / d_in_im; no other overlap.
  * Single-pass plans (1D, N <= 32768; 2D images of up to 16384 points) run one
- * launch; other plans stage through an interleaved buffer the plan allocates
- * at its first split call (synchronously: that first call is refused with
- * FG_ERR_INVALID_ARGUMENT, before any allocation, when `stream` is being
- * captured).
+ * launch; chunked multi-launch plans of 2^18 elements or more (2D: up to 1024
+ * rows) read and write the split arrays in their first and last passes, the
+ * other plans interleave into a staging buffer, run there and deinterleave
+ * (two more launches).  What either needs is allocated at the plan's first
+ * split call (synchronously: that first call of a multi-launch plan is
+ * refused with FG_ERR_INVALID_ARGUMENT, before any allocation, when `stream`
+ * is being captured).
  * Stream-ordered, asynchronous. */
 FG_API int fg_fft_exec_split(fg_fft_plan_t plan, const void *d_in_re, const void *d_in_im,
                              void *d_out_re, void *d_out_im, int direction, int normalize,
@@ -311,7 +314,9 @@ FG_API int fg_fft_exec_split(fg_fft_plan_t plan, const void *d_in_re, const void
  * from fg_device_open until the process ends, instead of the plan's lazily
  * allocated buffer; a plan whose batch needs more staging (8 bytes per
  * element of batch * elements) is refused with FG_ERR_INVALID_ARGUMENT.
- * Single-pass plans need no staging and run as fg_fft_exec_split does.
+ * Single-pass plans need no staging and run as fg_fft_exec_split does; 1D
+ * plans whose end passes read and write the split arrays stage nothing, but
+ * are bounded and take turns like the others.
  * Same results as fg_fft_exec_split, bit for bit (so, for the 2D plans named
  * there, the in-place interleaved execution's bits).  All callers on one GPU
  * share its scratch area, which keeps the last call's contents.  Outside
