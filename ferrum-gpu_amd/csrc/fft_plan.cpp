@@ -248,6 +248,37 @@ bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise) {
     return (g == 16 && (log_l == 9 || log_l == 10)) || (g == 32 && log_l == 8);
 }
 
+bool loads_cached(uint64_t bytes, uint64_t limit) {
+    // A first pass reads its input through the caches when the input is small
+    // enough to be in them still (the caller has often just written it); a
+    // streamed load does not fill the Infinity Cache, and hits in it are
+    // served at less than its rate.  Outputs are streamed at every size:
+    // cached stores displace the inputs and lost everywhere above 4 MiB (N =
+    // 1024, 16 MiB: 6.8 -> 8.8 us).  Measured on gfx950 over three input /
+    // output pairs in turn, us per execution, streamed / cached loads:
+    //  * 1D single pass up to 4096 points, limit 80 MiB: N = 16 8 MiB 7.0 /
+    //    4.0, 64 MiB 26.7 / 20.7; N = 1024 8 MiB 5.7 / 4.4, 16 MiB 7.2 / 7.1,
+    //    64 MiB 24.5 / 21.1, 80 MiB 30.3 / 25.7, 96 MiB 34.4 / 35.1; N = 4096
+    //    8 MiB 6.0 / 5.0, 16 MiB 7.6 / 7.7, 48 MiB 21.0 / 17.1, 96 MiB 36.4 /
+    //    37.0.  Over 24 pairs (no input left in a cache) N = 1024 32 MiB 12.1
+    //    / 12.5, N = 64 32 MiB 14.2 / 14.0.
+    //  * 8192 .. 32768 points, limit 16 MiB: 8192 8 MiB 9.2 / 8.6, 24 MiB
+    //    12.6 / 13.5; 32768 4 MiB 21.7 / 19.6, 16 MiB 22.5 / 21.1, 32 MiB
+    //    24.4 / 26.0.
+    //  * 2D one pass, limit 80 MiB: 64 x 64 8 MiB 7.7 / 6.7, 32 MiB 14.9 /
+    //    14.9, 80 MiB 34.4 / 27.6; 128 x 128 32 MiB 21.8 / 20.2.
+    //  * 2D row passes, limit 64 MiB: 512 x 512 x 3 12.1 / 10.7, 1024 x 1024
+    //    15.2 / 13.2, 256 x 256 x 64 24.1 / 22.6, 1024 x 1024 x 8 (64 MiB)
+    //    49.0 / 48.5, x 12 69.9 / 71.5.
+    //  * 1D multi-pass, limit 96 MiB: 48 MiB 2^16 38.3 / 33.5, 2^18 42.9 /
+    //    38.5, 2^20 46.2 / 41.6; 64 MiB 45.9 / 42.0, 49.3 / 46.0, 53.6 /
+    //    49.6, 2^23 67.1 / 62.5; 96 MiB 68.0 / 67.4, 75.8 / 71.4, 79.6 /
+    //    75.7; 128 MiB 2^16 86.5 / 88.8, 2^24 128.2 / 131.2.  32 MiB where
+    //    the last pass stores through the caches too (the 8-row tiles of 512
+    //    points): 2^17 32 MiB 28.1 / 27.7, 40 MiB 32.3 / 34.1.
+    return bytes <= limit;
+}
+
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
     // A launch in the pass's own tiles of G columns that would leave CUs idle,
     // or hold them at less than one round of narrower tiles, takes the
@@ -509,6 +540,7 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = p->steps_[0].name;
         p->split_fn_ = HipBackend::get_kernel(mod, (p->main_kernel_ + "_split").c_str());
         p->pw_ = Pointwise(mod);
+        p->load_cached_ = batch <= (1u << 24) && loads_cached((8ull * batch) << log_n, (log_n <= 12 ? 80ull : 16ull) << 20);
         p->fit_launches();
         return p;
     }
@@ -578,17 +610,7 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         t.ocs = 1;
         t.oes = N / L;
         p->add_tile(mod, log_l, g, true, t, (uint64_t)t.t0n * t.t1n, Buf::Work, Buf::Out, p->policy(P - 1, P));
-        // A plan of one chunk whose input, workspace and output fit the
-        // Infinity Cache together loads its input through it (the caller has
-        // often just written it; a streamed load neither fills the cache nor
-        // is served at its rate).  Measured on gfx950 over three alternating
-        // input / output pairs, us per execution, streamed / cached loads: 48
-        // MiB 2^16 38.3 / 33.5, 2^18 42.9 / 38.5, 2^20 46.2 / 41.6; 64 MiB
-        // 45.9 / 42.0, 49.3 / 46.0, 53.6 / 49.6, 2^23 67.1 / 62.5; 96 MiB 68.0
-        // / 67.4, 75.8 / 71.4, 79.6 / 75.7; 128 MiB 2^16 86.5 / 88.8, 2^24
-        // 128.2 / 131.2.  The 8-row last pass of 512 points stores through
-        // the caches too: 2^17 32 MiB 28.1 / 27.7, 40 MiB 32.3 / 34.1.
-        p->load_cached_ = p->cached_ && p->chunks() == 1 && 8ull * N * batch <= (g < 16 ? 32ull << 20 : 96ull << 20);
+        p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * N * batch, (g < 16 ? 32ull : 96ull) << 20);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -639,6 +661,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = s.name;
         p->split_fn_ = HipBackend::get_kernel(mod, (s.name + "_split").c_str());
         p->pw_ = Pointwise(mod);
+        p->load_cached_ = batch <= (1u << 24) && loads_cached(8ull * RC * batch, 80ull << 20);
         p->fit_launches();
         return p;
     }
@@ -651,6 +674,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
     // 256 324 -> 315, 1024 x 2048 378 -> 350, 32 x 1024 336 -> 314), 128 x
     // 2048 / 4096 and 512 x 4096 0.6 .. 1.3 % slower.
     p->choose_chunk(false);
+    p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * RC * batch, 64ull << 20);
     if (split) p->work_ = dev.alloc<Cf32>(RC * p->chunk_);
     // Row pass (the reference's K1 row FFT, py lib.rs:325-336): R rows of C per image.
     p->add_stockham(mod, log_cols, R, Buf::In, split ? Buf::Work : Buf::Out, p->policy(0, npass));
@@ -858,6 +882,7 @@ void FftPlan::run(const std::vector<Step>& steps, const Arrays& a, Direction dir
             uint32_t flags = 0;
             if (inverse && i == 0) flags |= FG_PASS_CONJ_IN;
             if (inverse && i + 1 == steps.size()) flags |= FG_PASS_CONJ_SCALE_OUT;
+            if (i == 0 && load_cached_) flags |= FG_PASS_LOAD_CACHED;
             void* args[9];
             size_t n = 0;
             // Input and output: one interleaved pointer each, or re and im.
@@ -916,8 +941,6 @@ void FftPlan::run(const std::vector<Step>& steps, const Arrays& a, Direction dir
                     g.tw0 /= k;
                     g.flags |= w << FG_PASS_WIDTH_SHIFT;
                     block = Dim3((w << s.log_l) / 16);
-                } else if (i == 0 && load_cached_) {
-                    g.flags |= FG_PASS_LOAD_CACHED;
                 }
                 if (w != s.width || line != 16) {
                     order = w < line ? FG_TILE_ORDER_LINE_GROUPS : 0u;
@@ -961,7 +984,8 @@ void FftPlan::check_split(const void* in_re, const void* in_im, const void* out_
 void FftPlan::split_one_launch(const void* in_re, const void* in_im, void* out_re, void* out_im, Direction dir,
                                bool normalize, hipStream_t stream) const {
     const Step& s = steps_[0];  // the split twin has the same geometry and table
-    uint32_t flags = dir == Direction::Inverse ? (FG_PASS_CONJ_IN | FG_PASS_CONJ_SCALE_OUT) : 0u;
+    uint32_t flags = dir == Direction::Inverse ? FG_PASS_CONJ : 0u;
+    if (load_cached_) flags |= FG_PASS_LOAD_CACHED;
     float sc = scale_for(dir, normalize);
     const void* tw = s.tw;
     const void* twc = s.tw_cols;

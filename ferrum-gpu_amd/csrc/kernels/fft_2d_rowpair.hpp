@@ -85,7 +85,7 @@ __device__ __forceinline__ void fft2d_rowpair_body(const float2* __restrict__ in
     const uint64_t half = 1ull << (log_rows - 1);
     const uint64_t r = p & (half - 1);
     const uint64_t first = (p >> (log_rows - 1)) << log_rows;  // the image's first row
-    const InterleavedIOT<false, true> io{in, out};              // rows streamed in, outputs kept cached
+    const InterleavedIOT<true> io{in, out};              // rows streamed in, outputs kept cached
     const uint64_t row_in = first + r + (s ? half : 0);
     float2 x[Sh::E];
 #pragma unroll
@@ -155,7 +155,7 @@ __device__ __forceinline__ void fft2d_rowpair_fused_body(const float2* __restric
     const uint64_t half = 1ull << (log_rows - 1);
     const uint64_t r = p & (half - 1);
     const uint64_t first = (p >> (log_rows - 1)) << log_rows;
-    const InterleavedIOT<false, true> io{in, out};
+    const InterleavedIOT<true> io{in, out};
     const uint64_t row_in = first + r + (s ? half : 0);
     float2 x[H::E], y[H::E];
 #pragma unroll

@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "tile_geom.h"
+
 namespace fg {
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
@@ -169,38 +171,44 @@ __device__ __forceinline__ void gstore(float* p, float v) {
 // position p: i = f * N + p) is in[i] in the interleaved complex64 layout (the
 // reference's Complex32 arrays), or (re[i], im[i]) in the split layout: two f32
 // arrays, the reference's SoA kernels (kernels_body.rs:509-626).
-template <bool LOAD_CACHED, bool STORE_CACHED>
+// Loads take their cache policy where they are made (load_policy below).
+template <bool STORE_CACHED>
 struct InterleavedIOT {
     const float2* in;
     float2* out;
-    __device__ __forceinline__ float2 load(uint64_t i) const { return gload<LOAD_CACHED>(in + i); }
+    template <bool CACHED = false>
+    __device__ __forceinline__ float2 load(uint64_t i) const { return gload<CACHED>(in + i); }
     __device__ __forceinline__ void store(uint64_t i, float2 v) const { gstore<STORE_CACHED>(out + i, v); }
     // Element row + lane with `row` the same for the whole wave: a scalar base
     // plus a 32-bit lane offset, no 64-bit vector address per access.
+    template <bool CACHED = false>
     __device__ __forceinline__ float2 load_row(uint64_t row, uint32_t lane) const {
-        return gload<LOAD_CACHED>(reinterpret_cast<const float2*>(reinterpret_cast<const char*>(in + row) + lane * 8u));
+        return gload<CACHED>(reinterpret_cast<const float2*>(reinterpret_cast<const char*>(in + row) + lane * 8u));
     }
     __device__ __forceinline__ void store_row(uint64_t row, uint32_t lane, float2 v) const {
         gstore<STORE_CACHED>(reinterpret_cast<float2*>(reinterpret_cast<char*>(out + row) + lane * 8u), v);
     }
 };
-using InterleavedIO = InterleavedIOT<false, false>;
+using InterleavedIO = InterleavedIOT<false>;
 struct SplitIO {
     const float* in_re;
     const float* in_im;
     float* out_re;
     float* out_im;
+    template <bool CACHED = false>
     __device__ __forceinline__ float2 load(uint64_t i) const {
-        return make_float2(load_stream(in_re + i), load_stream(in_im + i));
+        return make_float2(gload<CACHED>(in_re + i), gload<CACHED>(in_im + i));
     }
     __device__ __forceinline__ void store(uint64_t i, float2 v) const {
         store_stream(out_re + i, v.x);
         store_stream(out_im + i, v.y);
     }
+    template <bool CACHED = false>
     __device__ __forceinline__ float2 load_row(uint64_t row, uint32_t lane) const {
         const uint32_t b = lane * 4u;
-        return make_float2(load_stream(reinterpret_cast<const float*>(reinterpret_cast<const char*>(in_re + row) + b)),
-                           load_stream(reinterpret_cast<const float*>(reinterpret_cast<const char*>(in_im + row) + b)));
+        return make_float2(
+            gload<CACHED>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(in_re + row) + b)),
+            gload<CACHED>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(in_im + row) + b)));
     }
     __device__ __forceinline__ void store_row(uint64_t row, uint32_t lane, float2 v) const {
         const uint32_t b = lane * 4u;
@@ -209,14 +217,28 @@ struct SplitIO {
     }
 };
 
+// Runs the loads of a first pass, policy::value = whether they go through the
+// caches (FG_PASS_LOAD_CACHED): one branch per workgroup around the loads
+// alone, so the transform is one copy of code (and of bits) for both.
+template <bool B>
+struct LoadPolicy {
+    static constexpr bool value = B;
+};
+template <class F>
+__device__ __forceinline__ void load_policy(uint32_t flags, F loads) {
+    if (__builtin_expect((flags & FG_PASS_LOAD_CACHED) == 0, 1)) loads(LoadPolicy<false>{});
+    else loads(LoadPolicy<true>{});
+}
+
 // Split in, interleaved out: the row pass of a 2D plan on the split layout,
 // whose output the column pass reads next (streamed in, stored cached).
 struct SplitInIO {
     const float* in_re;
     const float* in_im;
     float2* out;
+    template <bool CACHED = false>
     __device__ __forceinline__ float2 load(uint64_t i) const {
-        return make_float2(load_stream(in_re + i), load_stream(in_im + i));
+        return make_float2(gload<CACHED>(in_re + i), gload<CACHED>(in_im + i));
     }
     __device__ __forceinline__ void store(uint64_t i, float2 v) const { gstore<true>(out + i, v); }
 };

@@ -39,7 +39,7 @@ using namespace fg;
         fg_fft_n##LOGN##_sc(const float2* __restrict__ in, float2* __restrict__ out,           \
                             const float2* __restrict__ tw, uint64_t batch, float scale,       \
                             uint32_t flags) {                                                 \
-        fft_stockham_body<LOGN, LOGE, FPB>(InterleavedIOT<false, true>{in, out}, tw, batch,   \
+        fft_stockham_body<LOGN, LOGE, FPB>(InterleavedIOT<true>{in, out}, tw, batch,   \
                                            scale, flags);                                     \
     }
 
@@ -69,7 +69,7 @@ FG_STOCKHAM(9, 4, 2)     // N=512:  32 threads
     extern "C" __global__ __launch_bounds__(128) void fg_fft_n10_sc(                                \
         const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ tw,      \
         uint64_t batch, float scale, uint32_t flags) {                                              \
-        fft1024_x2_body(InterleavedIOT<false, true>{in, out}, tw, batch, scale, flags);             \
+        fft1024_x2_body(InterleavedIOT<true>{in, out}, tw, batch, scale, flags);             \
     }
 FG_STOCKHAM_X2_1024()
 FG_STOCKHAM(11, 4, 1)    // N=2048: 128 threads

@@ -118,7 +118,7 @@ __device__ __forceinline__ void copy_shape_rowpair_halves(const float2* __restri
     const uint64_t half = 1ull << (log_rows - 1);
     const uint64_t r = p & (half - 1);
     const uint64_t first = (p >> (log_rows - 1)) << log_rows;
-    const InterleavedIOT<false, true> io{in, out};
+    const InterleavedIOT<true> io{in, out};
     const uint64_t row_in = first + r + (s ? half : 0);
     float2 x[H::E];
 #pragma unroll

@@ -14,8 +14,9 @@ namespace fg {
 #define FG_PASS_CONJ_IN 1u        /* conjugate every element on load */
 #define FG_PASS_CONJ_SCALE_OUT 2u /* conjugate, then multiply by `scale`, on store */
 #define FG_PASS_CONJ (FG_PASS_CONJ_IN | FG_PASS_CONJ_SCALE_OUT)
-/* Tile passes that stream their input in: load it through the caches instead
- * (a plan's only chunk, small enough to stay in the Infinity Cache). */
+/* Kernels that stream their input in: load it through the caches instead (a
+ * plan's first pass over an input small enough to stay in the Infinity
+ * Cache; loads_cached in fft_plan.cpp). */
 #define FG_PASS_LOAD_CACHED 4u
 /* Halves tile passes: flags >> FG_PASS_WIDTH_SHIFT is the columns per
  * workgroup of a launch in the kernel's narrow form (fft_tile_halves_pass),
