@@ -511,26 +511,27 @@ FG_TILE_SPLIT_OUT16(9, 8, r, true)
 // fg_<op>_vec: 16-byte accesses (every pointer 16-byte aligned; W elements
 // per thread step: 2 on interleaved streams, 4 for cmul_split); fg_<op>_elem:
 // one element per thread step, any alignment.  n is the number of complex
-// elements.  256-thread workgroups, grid-stride.
+// elements; flags: FG_PASS_LOAD_CACHED or 0.  256-thread workgroups,
+// grid-stride.
 #include "pointwise.hpp"
 
-#define FG_POINTWISE(SUFFIX, WC, WS)                                                                  \
-    extern "C" __global__ __launch_bounds__(256) void fg_cmul_c64_##SUFFIX(                          \
-        const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out, uint64_t n) { \
-        cmul_c64_body<WC>(a, b, out, n);                                                              \
-    }                                                                                                 \
-    extern "C" __global__ __launch_bounds__(256) void fg_cmul_split_##SUFFIX(                        \
-        const float* __restrict__ a_re, const float* __restrict__ a_im, const float* __restrict__ b_re, \
-        const float* __restrict__ b_im, float* __restrict__ o_re, float* __restrict__ o_im, uint64_t n) { \
-        cmul_split_body<WS>(a_re, a_im, b_re, b_im, o_re, o_im, n);                                   \
-    }                                                                                                 \
-    extern "C" __global__ __launch_bounds__(256) void fg_deinterleave_c64_##SUFFIX(                  \
-        const float* __restrict__ in, float* __restrict__ re, float* __restrict__ im, uint64_t n) {   \
-        deinterleave_body<WC>(in, re, im, n);                                                         \
-    }                                                                                                 \
-    extern "C" __global__ __launch_bounds__(256) void fg_interleave_c64_##SUFFIX(                    \
-        const float* __restrict__ re, const float* __restrict__ im, float* __restrict__ out, uint64_t n) { \
-        interleave_body<WC>(re, im, out, n);                                                          \
+#define FG_POINTWISE(SUFFIX, WC, WS)                                                                                       \
+    extern "C" __global__ __launch_bounds__(256) void fg_cmul_c64_##SUFFIX(                                                \
+        const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out, uint64_t n, uint32_t flags) {   \
+        load_policy(flags, [&](auto p) { cmul_c64_body<WC, p.value>(a, b, out, n); });                                     \
+    }                                                                                                                      \
+    extern "C" __global__ __launch_bounds__(256) void fg_cmul_split_##SUFFIX(                                              \
+        const float* __restrict__ a_re, const float* __restrict__ a_im, const float* __restrict__ b_re,                    \
+        const float* __restrict__ b_im, float* __restrict__ o_re, float* __restrict__ o_im, uint64_t n, uint32_t flags) {  \
+        load_policy(flags, [&](auto p) { cmul_split_body<WS, p.value>(a_re, a_im, b_re, b_im, o_re, o_im, n); });          \
+    }                                                                                                                      \
+    extern "C" __global__ __launch_bounds__(256) void fg_deinterleave_c64_##SUFFIX(                                        \
+        const float* __restrict__ in, float* __restrict__ re, float* __restrict__ im, uint64_t n, uint32_t flags) {        \
+        load_policy(flags, [&](auto p) { deinterleave_body<WC, p.value>(in, re, im, n); });                                \
+    }                                                                                                                      \
+    extern "C" __global__ __launch_bounds__(256) void fg_interleave_c64_##SUFFIX(                                          \
+        const float* __restrict__ re, const float* __restrict__ im, float* __restrict__ out, uint64_t n, uint32_t flags) { \
+        load_policy(flags, [&](auto p) { interleave_body<WC, p.value>(re, im, out, n); });                                 \
     }
 
 FG_POINTWISE(vec, 2, 4)

@@ -4,6 +4,7 @@ the same transforms at the head of a batch above it, in both layouts, and
 agrees with numpy in double precision; ragged last workgroups included."""
 
 import numpy as np
+import oracle
 import pytest
 
 from conftest import normal_c64, rel_l2
@@ -68,3 +69,75 @@ def test_cached_and_streamed_loads_give_the_same_bits(gpu_device, log_rows, log_
             assert np.array_equal(s.view(np.uint32), np.ascontiguousarray(part).view(np.uint32))
     p_small.destroy()
     p_big.destroy()
+
+
+# Elements at the edges of the ranges that load through the caches (load_flags,
+# ferrum-gpu_amd/csrc/pointwise_ops.cpp), ragged against the 2 and 4 elements
+# per thread.
+M12, M40, M80 = 12 << 17, 40 << 17, 80 << 17
+
+
+@pytest.mark.parametrize("n", [M12 - 1, M12, M12 + 3, M40 - 1, M40])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_products_by_load_policy(gpu_device, n, shift):
+    """out = a * b bit for bit in both layouts and in place; shift = 1 takes
+    the element-wise kernels."""
+    from ferrum_gpu import pointwise
+    from ferrum_gpu.hip import DeviceBuffer
+
+    print(f"[case] products n={n} shift={shift}", flush=True)
+    rng = np.random.default_rng(n + shift)
+    a, b = normal_c64(rng, n), normal_c64(rng, n)
+    want = oracle.cmul_interleaved(a, b)
+    bufs = [DeviceBuffer(gpu_device, 8 * (n + 1)) for _ in range(3)]
+    pad = np.zeros(n + 1, np.complex64)
+
+    def put(buf, v):
+        pad[shift:shift + n] = v
+        buf.copy_from_host(pad)
+
+    def get(buf):
+        gpu_device.sync()
+        return buf.copy_to_host(np.empty_like(pad))[shift:shift + n]
+
+    put(bufs[0], a)
+    put(bufs[1], b)
+    pa, pb, po = (int(x.ptr) + 8 * shift for x in bufs)
+    pointwise.cmul(gpu_device, pa, pb, po, n)
+    assert np.array_equal(get(bufs[2]).view(np.uint32), want.view(np.uint32))
+    pointwise.cmul(gpu_device, pa, pb, pa, n)
+    assert np.array_equal(get(bufs[0]).view(np.uint32), want.view(np.uint32))
+    w_re, w_im = oracle.cmul_split(a.real.copy(), a.imag.copy(), b.real.copy(), b.imag.copy())
+    parts = [DeviceBuffer(gpu_device, 4 * (n + 1)) for _ in range(6)]
+    fpad = np.zeros(n + 1, np.float32)
+    for buf, v in zip(parts, (a.real, a.imag, b.real, b.imag)):
+        fpad[shift:shift + n] = v
+        buf.copy_from_host(fpad)
+    pointwise.cmul_split(gpu_device, *[int(x.ptr) + 4 * shift for x in parts], n)
+    gpu_device.sync()
+    for buf, w in ((parts[4], w_re), (parts[5], w_im)):
+        got = buf.copy_to_host(np.empty_like(fpad))[shift:shift + n]
+        assert np.array_equal(got.view(np.uint32), w.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [M12 - 1, M12 + 1, M80 - 1, M80])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_conversions_by_load_policy(gpu_device, n, shift):
+    from ferrum_gpu import pointwise
+    from ferrum_gpu.hip import DeviceBuffer
+
+    print(f"[case] conversions n={n} shift={shift}", flush=True)
+    x = np.zeros(n + 1, np.complex64)
+    x[shift:shift + n] = normal_c64(np.random.default_rng(n + 2 + shift), n)
+    src, back = DeviceBuffer(gpu_device, 8 * (n + 1)), DeviceBuffer(gpu_device, 8 * (n + 1))
+    re, im = DeviceBuffer(gpu_device, 4 * (n + 1)), DeviceBuffer(gpu_device, 4 * (n + 1))
+    src.copy_from_host(x)
+    ps, pb, pr, pi = int(src.ptr) + 8 * shift, int(back.ptr) + 8 * shift, int(re.ptr) + 4 * shift, int(im.ptr) + 4 * shift
+    pointwise.deinterleave(gpu_device, ps, pr, pi, n)
+    pointwise.interleave(gpu_device, pr, pi, pb, n)
+    gpu_device.sync()
+    for buf, part in ((re, x.real), (im, x.imag)):
+        got = buf.copy_to_host(np.empty(n + 1, np.float32))[shift:shift + n]
+        assert np.array_equal(got.view(np.uint32), np.ascontiguousarray(part[shift:shift + n]).view(np.uint32))
+    got = back.copy_to_host(np.empty_like(x))[shift:shift + n]
+    assert np.array_equal(got.view(np.uint32), x[shift:shift + n].view(np.uint32))
