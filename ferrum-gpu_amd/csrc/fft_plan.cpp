@@ -254,29 +254,56 @@ bool loads_cached(uint64_t bytes, uint64_t limit) {
     // streamed load does not fill the Infinity Cache, and hits in it are
     // served at less than its rate.  Outputs are streamed at every size:
     // cached stores displace the inputs and lost everywhere above 4 MiB (N =
-    // 1024, 16 MiB: 6.8 -> 8.8 us).  Measured on gfx950 over three input /
-    // output pairs in turn, us per execution, streamed / cached loads:
-    //  * 1D single pass up to 4096 points, limit 80 MiB: N = 16 8 MiB 7.0 /
-    //    4.0, 64 MiB 26.7 / 20.7; N = 1024 8 MiB 5.7 / 4.4, 16 MiB 7.2 / 7.1,
-    //    64 MiB 24.5 / 21.1, 80 MiB 30.3 / 25.7, 96 MiB 34.4 / 35.1; N = 4096
-    //    8 MiB 6.0 / 5.0, 16 MiB 7.6 / 7.7, 48 MiB 21.0 / 17.1, 96 MiB 36.4 /
-    //    37.0.  Over 24 pairs (no input left in a cache) N = 1024 32 MiB 12.1
-    //    / 12.5, N = 64 32 MiB 14.2 / 14.0.
-    //  * 8192 .. 32768 points, limit 16 MiB: 8192 8 MiB 9.2 / 8.6, 24 MiB
+    // 1024, 16 MiB: 6.8 -> 8.8 us).  Each limit is the size up to which neither
+    // kind of caller loses: three input / output pairs in turn ("fw"), and
+    // three transforms there and back in turn ("rt", per execution, twice the
+    // inputs, half of them just streamed out).  Measured on gfx950, us per
+    // execution, streamed / cached loads:
+    //  * 1D single pass up to 4096 points, limit 44 MiB
+    //    (single_pass_loads_cached has the sizes within it that stream): N =
+    //    64 40 MiB fw 15.5 / 13.3, rt 16.1 / 15.1, 48 MiB 18.5 / 15.6, 19.0 /
+    //    19.4; N = 256 40 MiB 15.6 / 13.0, 15.8 / 14.6, 64 MiB 23.3 / 19.8,
+    //    23.6 / 24.4; N = 1024 40 MiB 17.0 / 13.7, 17.5 / 15.3, 48 MiB 19.2 /
+    //    16.4, 19.6 / 19.9; N = 4096 40 MiB 17.7 / 14.1, 18.1 / 16.1, 64 MiB
+    //    25.1 / 21.0, 25.4 / 26.0; N = 16 8 MiB fw 5.2 / 3.8.
+    //  * 8192 .. 32768 points, limit 16 MiB: 8192 8 MiB fw 9.2 / 8.6, 24 MiB
     //    12.6 / 13.5; 32768 4 MiB 21.7 / 19.6, 16 MiB 22.5 / 21.1, 32 MiB
     //    24.4 / 26.0.
-    //  * 2D one pass, limit 80 MiB: 64 x 64 8 MiB 7.7 / 6.7, 32 MiB 14.9 /
-    //    14.9, 80 MiB 34.4 / 27.6; 128 x 128 32 MiB 21.8 / 20.2.
-    //  * 2D row passes, limit 64 MiB: 512 x 512 x 3 12.1 / 10.7, 1024 x 1024
-    //    15.2 / 13.2, 256 x 256 x 64 24.1 / 22.6, 1024 x 1024 x 8 (64 MiB)
-    //    49.0 / 48.5, x 12 69.9 / 71.5.
-    //  * 1D multi-pass, limit 96 MiB: 48 MiB 2^16 38.3 / 33.5, 2^18 42.9 /
-    //    38.5, 2^20 46.2 / 41.6; 64 MiB 45.9 / 42.0, 49.3 / 46.0, 53.6 /
-    //    49.6, 2^23 67.1 / 62.5; 96 MiB 68.0 / 67.4, 75.8 / 71.4, 79.6 /
-    //    75.7; 128 MiB 2^16 86.5 / 88.8, 2^24 128.2 / 131.2.  32 MiB where
-    //    the last pass stores through the caches too (the 8-row tiles of 512
-    //    points): 2^17 32 MiB 28.1 / 27.7, 40 MiB 32.3 / 34.1.
+    //  * 2D one pass, limit 24 MiB: 64 x 64 8 MiB fw 7.7 / 6.7, 32 MiB 14.0 /
+    //    14.5, rt 14.5 / 14.8, 48 MiB 17.7 / 18.0, 18.1 / 18.5; 128 x 128 48
+    //    MiB 25.0 / 24.5, 25.2 / 25.6.
+    //  * 2D row passes, limit 40 MiB: 512 x 512 x 3 fw 12.1 / 10.7, 256 x 256
+    //    24 MiB 18.8 / 18.3, rt 18.5 / 18.2, 32 MiB 24.2 / 21.8, 23.3 / 23.2,
+    //    48 MiB 35.0 / 32.4, 34.6 / 35.1; 1024 x 1024 32 MiB 26.1 / 25.3, 25.8
+    //    / 26.0.
+    //  * 1D multi-pass, limit 56 MiB, 80 for 2^18 .. 2^20 points: 2^16 48 MiB
+    //    fw 38.8 / 33.5, rt 39.1 / 35.5, 64 MiB 46.3 / 41.7, 46.3 / 47.6; 2^18
+    //    64 MiB 48.9 / 45.1, 48.1 / 47.6; 2^20 64 MiB 51.7 / 47.7, 52.3 /
+    //    50.2, 96 MiB 75.6 / 74.5, 76.9 / 77.7; 2^23 64 MiB 67.4 / 62.3, 66.8 /
+    //    68.0.  32 MiB where the last pass stores through the caches too (the
+    //    8-row tiles of 512 points): 2^17 32 MiB fw 28.1 / 27.7, 40 MiB 32.3 /
+    //    34.1.
     return bytes <= limit;
+}
+
+bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes) {
+    // Between 12 MiB and `top`, inputs that other buffers' executions have
+    // pushed out of the L2s load faster streamed (from the Infinity Cache).
+    // Measured on gfx950, us per execution, streamed / cached, three input /
+    // output pairs in turn:
+    // N = 128 14 MiB 5.32 / 5.66, 18 MiB 6.19 / 6.50, 26 MiB 11.2 / 8.8; 256
+    // 18 MiB 6.58 / 7.21, 24 MiB 8.21 / 8.67, 26 MiB 9.9 / 9.2; 512 18 MiB
+    // 6.97 / 7.43, 22 MiB 7.70 / 8.27, 30 MiB 11.1 / 10.5; 2048 22 MiB 8.55 /
+    // 8.90, 30 MiB 10.43 / 10.67, 34 MiB 12.4 / 11.7; 4096 18 MiB 7.97 / 8.37,
+    // 26 MiB 9.98 / 9.70, 32 MiB 10.90 / 11.26, 34 MiB 15.0 / 12.9; 8 and 10
+    // MiB 2 .. 15 % faster cached, 1024 (two transforms per workgroup) within
+    // 2 % or faster cached at all of these but 28 MiB (10.1 / 10.4), N <= 64
+    // 6 .. 20 % faster cached.  One pair again and again, its input partly in
+    // the L2 that reads it, gains 3 .. 17 % cached here too; buffers in turn
+    // and inputs written elsewhere are the case the rule serves.
+    const uint64_t top = log_n < 7 || log_n == 10 ? 0 : log_n <= 9 ? 24ull << 20 : 32ull << 20;
+    if (log_n <= 12 && bytes > 12ull << 20 && bytes <= top) return false;
+    return loads_cached(bytes, (log_n <= 12 ? 44ull : 16ull) << 20);
 }
 
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
@@ -540,7 +567,7 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = p->steps_[0].name;
         p->split_fn_ = HipBackend::get_kernel(mod, (p->main_kernel_ + "_split").c_str());
         p->pw_ = Pointwise(mod);
-        p->load_cached_ = batch <= (1u << 24) && loads_cached((8ull * batch) << log_n, (log_n <= 12 ? 80ull : 16ull) << 20);
+        p->load_cached_ = batch <= (1u << 24) && single_pass_loads_cached(log_n, (8ull * batch) << log_n);
         p->fit_launches();
         return p;
     }
@@ -610,7 +637,8 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         t.ocs = 1;
         t.oes = N / L;
         p->add_tile(mod, log_l, g, true, t, (uint64_t)t.t0n * t.t1n, Buf::Work, Buf::Out, p->policy(P - 1, P));
-        p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * N * batch, (g < 16 ? 32ull : 96ull) << 20);
+        const uint64_t cached_limit = (g < 16 ? 32ull : log_n >= 18 && log_n <= 20 ? 80ull : 56ull) << 20;
+        p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * N * batch, cached_limit);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -661,7 +689,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = s.name;
         p->split_fn_ = HipBackend::get_kernel(mod, (s.name + "_split").c_str());
         p->pw_ = Pointwise(mod);
-        p->load_cached_ = batch <= (1u << 24) && loads_cached(8ull * RC * batch, 80ull << 20);
+        p->load_cached_ = batch <= (1u << 24) && loads_cached(8ull * RC * batch, 24ull << 20);
         p->fit_launches();
         return p;
     }
@@ -674,7 +702,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
     // 256 324 -> 315, 1024 x 2048 378 -> 350, 32 x 1024 336 -> 314), 128 x
     // 2048 / 4096 and 512 x 4096 0.6 .. 1.3 % slower.
     p->choose_chunk(false);
-    p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * RC * batch, 64ull << 20);
+    p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * RC * batch, 40ull << 20);
     if (split) p->work_ = dev.alloc<Cf32>(RC * p->chunk_);
     // Row pass (the reference's K1 row FFT, py lib.rs:325-336): R rows of C per image.
     p->add_stockham(mod, log_cols, R, Buf::In, split ? Buf::Work : Buf::Out, p->policy(0, npass));

@@ -284,6 +284,8 @@ bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
 // Whether a plan whose whole input is `bytes` loads it through the caches,
 // given its kind's limit.
 bool loads_cached(uint64_t bytes, uint64_t limit);
+// The same for single-pass 1D plans of 2^log_n points.
+bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes);
 // Columns per workgroup of a launch of `tiles` tiles of a pass (2^log_l points, g columns per tile) in its narrow form; 0: its own tiles.
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count);
 // Whether the column FFT of an image with 2^log_rows rows runs as two passes.

@@ -20,7 +20,7 @@ TOL = 8e-7
 # (log_rows, log_n, MiB below, MiB above): below is large enough for the
 # throughput kernels (the latency ones of 256, 1024 and 4096 points have
 # another radix list).
-CASES = [(0, n, 17, 82) for n in range(2, 13)] + [(0, n, 12, 18) for n in (13, 14, 15)] + \
+CASES = [(0, n, 40, 82) for n in range(2, 13)] + [(0, 9, 20, 30), (0, 12, 30, 36)] + [(0, n, 12, 18) for n in (13, 14, 15)] + \
     [(4, 4, 9, 82), (4, 6, 9, 82), (5, 5, 9, 82), (5, 6, 9, 82), (6, 6, 9, 82), (7, 7, 9, 82), (4, 10, 9, 82),
      (6, 9, 40, 66), (10, 10, 40, 72)]
 
