@@ -219,15 +219,24 @@ struct SplitIO {
 
 // Runs the loads of a first pass, policy::value = whether they go through the
 // caches (FG_PASS_LOAD_CACHED): one branch per workgroup around the loads
-// alone, so the transform is one copy of code (and of bits) for both.
+// alone, so the transform is one copy of code (and of bits) for both.  The two
+// branches differ in the cache hint alone, which the compiler drops to merge
+// equal loads (the f32 loads of the split layout: every size of most split
+// kernels loaded through the caches); the empty asm statements, in one branch
+// only, keep it from hoisting loads above the branch or sinking them below.
 template <bool B>
 struct LoadPolicy {
     static constexpr bool value = B;
 };
 template <class F>
 __device__ __forceinline__ void load_policy(uint32_t flags, F loads) {
-    if (__builtin_expect((flags & FG_PASS_LOAD_CACHED) == 0, 1)) loads(LoadPolicy<false>{});
-    else loads(LoadPolicy<true>{});
+    if (__builtin_expect((flags & FG_PASS_LOAD_CACHED) == 0, 1)) {
+        asm volatile("; streamed loads");
+        loads(LoadPolicy<false>{});
+        asm volatile("; streamed loads end");
+    } else {
+        loads(LoadPolicy<true>{});
+    }
 }
 
 // Split in, interleaved out: the row pass of a 2D plan on the split layout,
