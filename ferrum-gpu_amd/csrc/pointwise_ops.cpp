@@ -34,11 +34,26 @@ bool overlap(const void* a, uint64_t abytes, const void* b, uint64_t bbytes) {
     return x < y + bbytes && y < x + abytes;
 }
 
-// FG_PASS_LOAD_CACHED for arrays of `from` MiB up to `limit`.
-uint32_t load_flags(uint64_t n, uint64_t from, uint64_t limit) {
+// The kernels' last argument: whether they load their inputs through the
+// caches, by the bytes of one complex array of n elements.  From 12 MiB up to
+// 40 MiB for a product (which reads two arrays) and 80 MiB for a conversion.
+// Below, a launch is bound by the host and streamed as before (a filter of one
+// 1024 x 1024 image, 8 MiB: 35.7 us streamed, 37.2 cached); above, the inputs
+// no longer fit the Infinity Cache beside the output.  Measured on gfx950, us
+// per launch, streamed / cached, the same buffers each time and three sets in
+// turn: cmul 16 MiB 7.6 / 6.7 and 9.0 / 8.4, 24 MiB 11.4 / 11.8 and 13.0 /
+// 11.9, 32 MiB 15.1 / 15.2 and 16.7 / 15.3, 48 MiB 22.6 / 21.7 and 24.1 /
+// 24.5, 64 MiB 30.0 / 28.4 and 31.3 / 34.3; interleave 16 MiB 6.4 / 4.9 and
+// 7.3 / 6.4, 24 MiB 8.9 / 5.2 and 9.9 / 8.5, 64 MiB 22.6 / 20.5 and 23.7 /
+// 20.6, 96 MiB 33.1 / 29.6 and 33.5 / 33.8; deinterleave 24 MiB 9.5 / 5.3 and
+// 9.9 / 8.4, 64 MiB 23.4 / 19.9 and 23.4 / 20.0.  A filter (transform,
+// product, inverse, in place) of 24 MiB of 1024 x 1024 images 61.9 / 58.6, 32
+// MiB of 512 x 512 73.0 / 69.0, one 2048 x 2048 image 73.5 / 70.9.
+uint32_t load_flags(uint64_t n, uint64_t limit) {
     const uint64_t mib = n >> 17;  // of 8 n bytes
-    return mib >= from && mib < limit ? FG_PASS_LOAD_CACHED : 0u;
+    return mib >= 12 && mib < limit ? FG_PASS_LOAD_CACHED : 0u;
 }
+constexpr uint64_t kProductMiB = 40, kConvertMiB = 80;
 
 void launch(const HipBackend::DeviceHandle& dev, hipStream_t stream, HipBackend::KernelHandle k, uint64_t n,
             int width, void** args) {
@@ -49,35 +64,6 @@ void launch(const HipBackend::DeviceHandle& dev, hipStream_t stream, HipBackend:
 }
 
 }  // namespace
-
-// The kernels' last argument: whether they load their inputs through the
-// caches, by the bytes of one complex array of n elements: from 13 to 40 MiB
-// for a product (which reads two arrays), from 12 to 80 MiB for a conversion.
-// Below, a launch is bound by the host; above, the inputs no longer fit the
-// Infinity Cache beside the output.  Measured on gfx950, us per launch,
-// streamed / cached, the same buffers each time, three sets in turn, and sets
-// last touched 1.2 GB of other traffic before ("cold"):
-//   product out of place  16 MiB 6.8 / 6.8, 9.2 / 8.5, 9.9 / 10.5
-//                         24 MiB 11.4 / 11.7, 13.1 / 11.9, 13.6 / 14.3
-//                         39 MiB 18.2 / 17.9, 20.1 / 18.2, 21.0 / 21.9
-//   product in place      12 MiB 5.1 / 5.1, 6.9 / 6.9, 7.9 / 9.1
-//                         16 MiB 7.6 / 5.0, 9.2 / 8.6, 9.8 / 11.4
-//                         20 MiB 9.6 / 10.1, 11.0 / 10.2, 11.6 / 13.1
-//                         32 MiB 14.6 / 15.3, 16.9 / 15.3, 17.2 / 19.4
-//   interleave            16 MiB 5.0 / 5.0, 6.6 / 6.6, 7.8 / 8.2
-//                         24 MiB 6.4 / 5.2, 9.7 / 8.9, 10.5 / 11.1
-//                         32 MiB 9.2 / 10.3, 12.6 / 11.3, 13.2 / 13.8
-//                         64 MiB 21.8 / 20.5, 23.1 / 20.0, 23.5 / 24.1
-// (deinterleave within 4 % of interleave's ratios).  Arrays that the calls
-// before have left in the Infinity Cache gain, cold ones lose.  A filter
-// (transform, product, inverse, in place) of a multi-launch plan: 12 MiB of
-// 512 x 512 images 45.6 / 46.6, 42.4 / 43.3, 43.9 / 45.1, 24 MiB of 1024 x
-// 1024 64.1 / 60.7, 62.3 / 59.0, 64.7 / 63.5, 32 MiB of 512 x 512 72.3 / 65.2,
-// 72.2 / 67.8, 75.6 / 69.5; of a single-pass plan, whose output streams past
-// the caches: 23 MiB of 256 points 28.2 / 32.5, 30.2 / 32.8, 30.8 / 34.0, 35
-// MiB of 1024 points 45.7 / 42.9, 46.1 / 45.9, 52.2 / 48.5.
-uint32_t product_flags(uint64_t n) { return load_flags(n, 13, 40); }
-uint32_t convert_flags(uint64_t n) { return load_flags(n, 12, 80); }
 
 Pointwise::Pointwise(const HipBackend::Module& mod) {
     for (int v = 0; v < 2; ++v) {
@@ -102,7 +88,7 @@ void Pointwise::cmul_c64(const HipBackend::DeviceHandle& dev, const void* a, con
     for (const void* x : {a, b})
         if (x != out && overlap(out, 8 * n, x, 8 * n)) invalid("cmul_c64: out partially overlaps an input");
     const int v = aligned16({a, b, out}) ? 1 : 0;
-    uint32_t flags = product_flags(n);
+    uint32_t flags = load_flags(n, kProductMiB);
     void* args[] = {(void*)&a, (void*)&b, &out, &n, &flags};
     launch(dev, stream, cmul_c64_[v], n, v ? 2 : 1, args);
 }
@@ -125,7 +111,7 @@ void Pointwise::cmul_split(const HipBackend::DeviceHandle& dev, const void* a_re
     }
     if (overlap(o_re, nb, o_im, nb)) invalid("cmul_split: o_re and o_im overlap");
     const int v = aligned16({a_re, a_im, b_re, b_im, o_re, o_im}) ? 1 : 0;
-    uint32_t flags = product_flags(n);
+    uint32_t flags = load_flags(n, kProductMiB);
     void* args[] = {(void*)&a_re, (void*)&a_im, (void*)&b_re, (void*)&b_im, &o_re, &o_im, &n, &flags};
     launch(dev, stream, cmul_split_[v], n, v ? 4 : 1, args);
 }
@@ -137,7 +123,7 @@ void Pointwise::deinterleave(const HipBackend::DeviceHandle& dev, const void* in
     if (overlap(in, 8 * n, re, 4 * n) || overlap(in, 8 * n, im, 4 * n) || overlap(re, 4 * n, im, 4 * n))
         invalid("deinterleave: buffers overlap");
     const int v = aligned16({in, re, im}) ? 1 : 0;
-    uint32_t flags = convert_flags(n);
+    uint32_t flags = load_flags(n, kConvertMiB);
     void* args[] = {(void*)&in, &re, &im, &n, &flags};
     launch(dev, stream, deinterleave_[v], n, v ? 2 : 1, args);
 }
@@ -148,7 +134,7 @@ void Pointwise::interleave(const HipBackend::DeviceHandle& dev, const void* re, 
     need_ptrs("interleave", {re, im, out});
     if (overlap(out, 8 * n, re, 4 * n) || overlap(out, 8 * n, im, 4 * n)) invalid("interleave: buffers overlap");
     const int v = aligned16({re, im, out}) ? 1 : 0;
-    uint32_t flags = convert_flags(n);
+    uint32_t flags = load_flags(n, kConvertMiB);
     void* args[] = {(void*)&re, (void*)&im, &out, &n, &flags};
     launch(dev, stream, interleave_[v], n, v ? 2 : 1, args);
 }

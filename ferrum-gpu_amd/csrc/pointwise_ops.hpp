@@ -22,10 +22,6 @@
 
 namespace fg {
 
-// The flags argument of a product's / a conversion's kernel for n elements.
-uint32_t product_flags(uint64_t n);
-uint32_t convert_flags(uint64_t n);
-
 class Pointwise {
 public:
     explicit Pointwise(const HipBackend::Module& mod);

@@ -71,13 +71,13 @@ def test_cached_and_streamed_loads_give_the_same_bits(gpu_device, log_rows, log_
     p_big.destroy()
 
 
-# Elements at the edges of the ranges that load through the caches (product_flags
-# and convert_flags, ferrum-gpu_amd/csrc/pointwise_ops.cpp), ragged against the 2
-# and 4 elements per thread.
-M12, M13, M40, M80 = 12 << 17, 13 << 17, 40 << 17, 80 << 17
+# Elements at the edges of the ranges that load through the caches (load_flags,
+# ferrum-gpu_amd/csrc/pointwise_ops.cpp), ragged against the 2 and 4 elements
+# per thread.
+M12, M40, M80 = 12 << 17, 40 << 17, 80 << 17
 
 
-@pytest.mark.parametrize("n", [M13 - 1, M13, M13 + 3, M40 - 1, M40])
+@pytest.mark.parametrize("n", [M12 - 1, M12, M12 + 3, M40 - 1, M40])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_products_by_load_policy(gpu_device, n, shift):
     """out = a * b bit for bit in both layouts and in place; shift = 1 takes
