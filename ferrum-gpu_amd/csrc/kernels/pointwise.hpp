@@ -9,9 +9,8 @@
 // deinterleave / interleave take 8 bytes per lane.  The host picks them when
 // every pointer is 16-byte aligned.  W = 1 goes element by element for any
 // complex64 / f32 alignment.  CACHED loads the inputs through the caches, for
-// arrays small enough to be in them still (load_flags in pointwise_ops.cpp:
-// interleave at 24 MiB 8.9 -> 5.2 us, cmul at 32 MiB 16.7 -> 15.3); outputs
-// are streamed.  The complex product is evaluated as written,
+// arrays small enough to be in them still (load_flags in pointwise_ops.cpp has
+// the ranges and what they measured); outputs are streamed.  The complex product is evaluated as written,
 // re = ar*br - ai*bi, im = ar*bi + ai*br, with no fused multiply-add, so
 // results equal the reference's f32 arithmetic (Rust does not contract) bit
 // for bit.

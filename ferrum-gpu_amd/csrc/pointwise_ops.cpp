@@ -37,18 +37,35 @@ bool overlap(const void* a, uint64_t abytes, const void* b, uint64_t bbytes) {
 // The kernels' last argument: whether they load their inputs through the
 // caches, by the bytes of one complex array of n elements.  From 12 MiB up to
 // 40 MiB for a product (which reads two arrays) and 80 MiB for a conversion.
-// Below, a launch is bound by the host and streamed as before (a filter of one
-// 1024 x 1024 image, 8 MiB: 35.7 us streamed, 37.2 cached); above, the inputs
-// no longer fit the Infinity Cache beside the output.  Measured on gfx950, us
-// per launch, streamed / cached, the same buffers each time and three sets in
-// turn: cmul 16 MiB 7.6 / 6.7 and 9.0 / 8.4, 24 MiB 11.4 / 11.8 and 13.0 /
-// 11.9, 32 MiB 15.1 / 15.2 and 16.7 / 15.3, 48 MiB 22.6 / 21.7 and 24.1 /
-// 24.5, 64 MiB 30.0 / 28.4 and 31.3 / 34.3; interleave 16 MiB 6.4 / 4.9 and
-// 7.3 / 6.4, 24 MiB 8.9 / 5.2 and 9.9 / 8.5, 64 MiB 22.6 / 20.5 and 23.7 /
-// 20.6, 96 MiB 33.1 / 29.6 and 33.5 / 33.8; deinterleave 24 MiB 9.5 / 5.3 and
-// 9.9 / 8.4, 64 MiB 23.4 / 19.9 and 23.4 / 20.0.  A filter (transform,
-// product, inverse, in place) of 24 MiB of 1024 x 1024 images 61.9 / 58.6, 32
-// MiB of 512 x 512 73.0 / 69.0, one 2048 x 2048 image 73.5 / 70.9.
+// Below, a launch is bound by the host; above, the inputs no longer fit the
+// Infinity Cache beside the output.  Measured on gfx950: us per launch with
+// streamed loads and the change, in percent, with cached ones, for the same
+// buffers each time, three sets in turn, and buffers last touched 1.2 GB of
+// other traffic before ("cold"); the caches are flushed between settings and
+// warmed by each setting itself:
+//                             the same  in turn    cold
+//   product, in place 12 MiB  7.5 -34   8.0 -13    8.1 +12
+//                     16 MiB  9.4 -47   9.8 -11    10.0 +14
+//                     32 MiB  17.1 -9   17.7 -14   17.6 +11
+//   out of place      16 MiB  9.3 -28   9.9 -12    10.1 +3
+//                     24 MiB  13.1 -9   13.7 -13   13.9 +3
+//                     36 MiB  18.9 -10  19.4 -11   19.4 +4
+//                     48 MiB  24.4 -11  25.0 +5    25.0 +5
+//   split             24 MiB  13.5 -8   14.7 -15   14.9 +5
+//   interleave        12 MiB  6.1 -20   6.4 -19    6.6 +2
+//                     24 MiB  10.3 -50  10.7 -16   10.9 +4
+//                     79 MiB  28.4 -13  28.6 -15   28.6 +2
+//   deinterleave      24 MiB  9.9 -47   10.3 -16   10.3 +5
+// (A product over the same 20 to 28 MiB arrays, just written and never
+// displaced, runs 3 to 7 % faster streamed.)  The product within a filter
+// (transform, product, inverse, in place) gains on multi-launch plans: 1024 x
+// 1024 24 MiB 63.9 -5, 62.3 -5, 64.7 -2, 512 x 512 32 MiB 73.0 -10, 72.9 -4,
+// 76.1 -8 (12 MiB 45.7 +2, 42.4 +2, 44.0 +2), 2^16 points 24 MiB 58.3 -6, 58.1
+// -6, 59.8 -4.  It loses on single-pass plans below about 30 MiB, whose
+// outputs were streamed out and are not in the caches: 256 points 23 MiB 30.8
+// +7, 30.9 +7, 31.1 +11, 1024 points 16 MiB 24.2 +5, 25.3 +5, 27.5 +5, 35 MiB
+// 48.7 -9, 47.0 -2, 52.4 -7.  A product does not know what wrote its inputs;
+// the range weighs these.
 uint32_t load_flags(uint64_t n, uint64_t limit) {
     const uint64_t mib = n >> 17;  // of 8 n bytes
     return mib >= 12 && mib < limit ? FG_PASS_LOAD_CACHED : 0u;
