@@ -195,7 +195,7 @@ __device__ __forceinline__ void fft2d_halves_body(const IO io, const float2* __r
     if (f >= batch || t >= H::T) return;
     stagger_lockstep_start<(H::HALF + H::HALF / 16) * 8, H::T>();  // 16384-point images
     float2 x[H::E], y[H::E];
-    load_policy(flags, [&](auto policy) {
+    load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
         for (int m = 0; m < H::E; ++m) x[m] = io.template load_row<policy.value>(f * H::N + H::T * m, t);
     });

@@ -115,7 +115,7 @@ __device__ __forceinline__ void fft2d_small_body(const IO io, const float2* __re
     // load's write beside it: 16 x 16 192.5 -> 176.0 us, 32 x 32 195.4 ->
     // 176.9, 16 x 64 193.3 -> 174.7).
     float2 in[S::E];
-    load_policy(flags, [&](auto policy) {
+    load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
         for (int j = 0; j < S::E; ++j) {
             const int e = tid + S::BLOCK * j;

@@ -176,6 +176,7 @@ template <bool STORE_CACHED>
 struct InterleavedIOT {
     const float2* in;
     float2* out;
+    static constexpr bool F32 = false;  // load_policy
     template <bool CACHED = false>
     __device__ __forceinline__ float2 load(uint64_t i) const { return gload<CACHED>(in + i); }
     __device__ __forceinline__ void store(uint64_t i, float2 v) const { gstore<STORE_CACHED>(out + i, v); }
@@ -195,6 +196,7 @@ struct SplitIO {
     const float* in_im;
     float* out_re;
     float* out_im;
+    static constexpr bool F32 = true;
     template <bool CACHED = false>
     __device__ __forceinline__ float2 load(uint64_t i) const {
         return make_float2(gload<CACHED>(in_re + i), gload<CACHED>(in_im + i));
@@ -219,21 +221,24 @@ struct SplitIO {
 
 // Runs the loads of a first pass, policy::value = whether they go through the
 // caches (FG_PASS_LOAD_CACHED): one branch per workgroup around the loads
-// alone, so the transform is one copy of code (and of bits) for both.  The two
-// branches differ in the cache hint alone, which the compiler drops to merge
-// equal loads (the f32 loads of the split layout: every size of most split
-// kernels loaded through the caches); the empty asm statements, in one branch
-// only, keep it from hoisting loads above the branch or sinking them below.
+// alone, so the transform is one copy of code (and of bits) for both.
+// F32 (the split layout): both branches make the same float loads, which
+// differ in the cache hint alone, and the compiler drops it to merge them
+// (most split kernels then loaded through the caches at every size).  The empty
+// asm statements, in one branch only, keep it from hoisting the loads above
+// the branch or sinking them below it.  Interleaved loads differ in type and
+// stay apart by themselves; the statements would cost them 2 to 3 % (N = 1024
+// at 24 to 34 MiB).
 template <bool B>
 struct LoadPolicy {
     static constexpr bool value = B;
 };
-template <class F>
+template <bool F32, class F>
 __device__ __forceinline__ void load_policy(uint32_t flags, F loads) {
     if (__builtin_expect((flags & FG_PASS_LOAD_CACHED) == 0, 1)) {
-        asm volatile("; streamed loads");
+        if constexpr (F32) asm volatile("; streamed loads");
         loads(LoadPolicy<false>{});
-        asm volatile("; streamed loads end");
+        if constexpr (F32) asm volatile("; streamed loads end");
     } else {
         loads(LoadPolicy<true>{});
     }
@@ -245,6 +250,7 @@ struct SplitInIO {
     const float* in_re;
     const float* in_im;
     float2* out;
+    static constexpr bool F32 = true;
     template <bool CACHED = false>
     __device__ __forceinline__ float2 load(uint64_t i) const {
         return make_float2(gload<CACHED>(in_re + i), gload<CACHED>(in_im + i));

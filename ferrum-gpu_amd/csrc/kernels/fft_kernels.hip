@@ -518,20 +518,20 @@ FG_TILE_SPLIT_OUT16(9, 8, r, true)
 #define FG_POINTWISE(SUFFIX, WC, WS)                                                                                       \
     extern "C" __global__ __launch_bounds__(256) void fg_cmul_c64_##SUFFIX(                                                \
         const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out, uint64_t n, uint32_t flags) {   \
-        load_policy(flags, [&](auto p) { cmul_c64_body<WC, p.value>(a, b, out, n); });                                     \
+        load_policy<false>(flags, [&](auto p) { cmul_c64_body<WC, p.value>(a, b, out, n); });                                     \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(256) void fg_cmul_split_##SUFFIX(                                              \
         const float* __restrict__ a_re, const float* __restrict__ a_im, const float* __restrict__ b_re,                    \
         const float* __restrict__ b_im, float* __restrict__ o_re, float* __restrict__ o_im, uint64_t n, uint32_t flags) {  \
-        load_policy(flags, [&](auto p) { cmul_split_body<WS, p.value>(a_re, a_im, b_re, b_im, o_re, o_im, n); });          \
+        load_policy<false>(flags, [&](auto p) { cmul_split_body<WS, p.value>(a_re, a_im, b_re, b_im, o_re, o_im, n); });          \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(256) void fg_deinterleave_c64_##SUFFIX(                                        \
         const float* __restrict__ in, float* __restrict__ re, float* __restrict__ im, uint64_t n, uint32_t flags) {        \
-        load_policy(flags, [&](auto p) { deinterleave_body<WC, p.value>(in, re, im, n); });                                \
+        load_policy<false>(flags, [&](auto p) { deinterleave_body<WC, p.value>(in, re, im, n); });                                \
     }                                                                                                                      \
     extern "C" __global__ __launch_bounds__(256) void fg_interleave_c64_##SUFFIX(                                          \
         const float* __restrict__ re, const float* __restrict__ im, float* __restrict__ out, uint64_t n, uint32_t flags) { \
-        load_policy(flags, [&](auto p) { interleave_body<WC, p.value>(re, im, out, n); });                                 \
+        load_policy<false>(flags, [&](auto p) { interleave_body<WC, p.value>(re, im, out, n); });                                 \
     }
 
 FG_POINTWISE(vec, 2, 4)

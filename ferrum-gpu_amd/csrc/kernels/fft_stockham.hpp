@@ -287,7 +287,7 @@ __device__ __forceinline__ void fft_stockham_body(const IO io, const float2* __r
         // All loads first, then the LDS writes: with each load's write beside
         // it the wave waited for every element in turn (N = 16 at 512 MiB
         // 179.6 -> 168.6 us, N = 32 179.8 -> 168.8, gfx950).
-        load_policy(flags, [&](auto policy) {
+        load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
             for (int j = 0; j < Sh::E; ++j) {
                 const int e = tid + BLOCK * j;  // element of the block's FPB*N
@@ -304,7 +304,7 @@ __device__ __forceinline__ void fft_stockham_body(const IO io, const float2* __r
         for (int m = 0; m < Sh::E; ++m) x[m] = lds_all[slot][lds_pos<>(t + Sh::T * m)];
         if constexpr (ONE_WAVE) wave_sync(); else __syncthreads();
     } else if (valid) {
-        load_policy(flags, [&](auto policy) {
+        load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
             for (int m = 0; m < Sh::E; ++m) x[m] = io.template load<policy.value>(f * Sh::N + t + Sh::T * m);
         });
@@ -458,7 +458,7 @@ __device__ __forceinline__ void fft_row_halves_body(const IO io, const float2* _
     if (f >= batch) return;  // uniform over the workgroup (the host launches batch of them)
     stagger_lockstep_start<(H::HALF + H::HALF / 16) * 8, H::T>();  // 16384 / 32768 points
     float2 x[H::E], y[H::E];
-    load_policy(flags, [&](auto policy) {
+    load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
         for (int m = 0; m < H::E; ++m) x[m] = io.template load_row<policy.value>(f * H::N + H::T * m, t);
     });
@@ -503,7 +503,7 @@ __device__ __forceinline__ void fft1024_x2_body(const IO io, const float2* __res
     const uint64_t f0 = (uint64_t)blockIdx.x * 2;
     const bool has1 = f0 + 1 < batch;  // the last workgroup may hold one transform
     float2 x[16];
-    load_policy(flags, [&](auto policy) {
+    load_policy<IO::F32>(flags, [&](auto policy) {
 #pragma unroll
         for (int f = 0; f < 2; ++f)
 #pragma unroll
