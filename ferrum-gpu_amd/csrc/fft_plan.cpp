@@ -248,62 +248,132 @@ bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise) {
     return (g == 16 && (log_l == 9 || log_l == 10)) || (g == 32 && log_l == 8);
 }
 
-bool loads_cached(uint64_t bytes, uint64_t limit) {
-    // A first pass reads its input through the caches when the input is small
-    // enough to be in them still (the caller has often just written it); a
-    // streamed load does not fill the Infinity Cache, and hits in it are
-    // served at less than its rate.  Outputs are streamed at every size:
-    // cached stores displace the inputs and lost everywhere above 4 MiB (N =
-    // 1024, 16 MiB: 6.8 -> 8.8 us).  Each limit is the size up to which neither
-    // kind of caller loses: three input / output pairs in turn ("fw"), and
-    // three transforms there and back in turn ("rt", per execution, twice the
-    // inputs, half of them just streamed out).  Measured on gfx950, us per
-    // execution, streamed / cached loads:
-    //  * 1D single pass up to 4096 points, limit 44 MiB
-    //    (single_pass_loads_cached has the sizes within it that stream): N =
-    //    64 40 MiB fw 15.5 / 13.3, rt 16.1 / 15.1, 48 MiB 18.5 / 15.6, 19.0 /
-    //    19.4; N = 256 40 MiB 15.6 / 13.0, 15.8 / 14.6, 64 MiB 23.3 / 19.8,
-    //    23.6 / 24.4; N = 1024 40 MiB 17.0 / 13.7, 17.5 / 15.3, 48 MiB 19.2 /
-    //    16.4, 19.6 / 19.9; N = 4096 40 MiB 17.7 / 14.1, 18.1 / 16.1, 64 MiB
-    //    25.1 / 21.0, 25.4 / 26.0; N = 16 8 MiB fw 5.2 / 3.8.
-    //  * 8192 .. 32768 points, limit 16 MiB: 8192 8 MiB fw 9.2 / 8.6, 24 MiB
-    //    12.6 / 13.5; 32768 4 MiB 21.7 / 19.6, 16 MiB 22.5 / 21.1, 32 MiB
-    //    24.4 / 26.0.
-    //  * 2D one pass, limit 24 MiB: 64 x 64 8 MiB fw 7.7 / 6.7, 32 MiB 14.0 /
-    //    14.5, rt 14.5 / 14.8, 48 MiB 17.7 / 18.0, 18.1 / 18.5; 128 x 128 48
-    //    MiB 25.0 / 24.5, 25.2 / 25.6.
-    //  * 2D row passes, limit 40 MiB: 512 x 512 x 3 fw 12.1 / 10.7, 256 x 256
-    //    24 MiB 18.8 / 18.3, rt 18.5 / 18.2, 32 MiB 24.2 / 21.8, 23.3 / 23.2,
-    //    48 MiB 35.0 / 32.4, 34.6 / 35.1; 1024 x 1024 32 MiB 26.1 / 25.3, 25.8
-    //    / 26.0.
-    //  * 1D multi-pass, limit 56 MiB, 80 for 2^18 .. 2^20 points: 2^16 48 MiB
-    //    fw 38.8 / 33.5, rt 39.1 / 35.5, 64 MiB 46.3 / 41.7, 46.3 / 47.6; 2^18
-    //    64 MiB 48.9 / 45.1, 48.1 / 47.6; 2^20 64 MiB 51.7 / 47.7, 52.3 /
-    //    50.2, 96 MiB 75.6 / 74.5, 76.9 / 77.7; 2^23 64 MiB 67.4 / 62.3, 66.8 /
-    //    68.0.  32 MiB where the last pass stores through the caches too (the
-    //    8-row tiles of 512 points): 2^17 32 MiB fw 28.1 / 27.7, 40 MiB 32.3 /
-    //    34.1.
-    return bytes <= limit;
-}
+// First passes load an input through the caches when it is small enough to be
+// in them still (the caller has often just written it); a streamed load does
+// not fill the Infinity Cache, and hits in it are served at less than its
+// rate.  Outputs are streamed at every size: cached stores displace the
+// inputs and lost everywhere above 4 MiB (N = 1024, 16 MiB: 6.8 -> 8.8 us).
+// The ranges below are measured on gfx950 with four kinds of caller: one pair
+// of buffers again and again ("one"), three pairs in turn ("turn"), three
+// transforms there and back ("back", per execution), and pairs last touched
+// 1.2 GB of other traffic before ("cold"); us per execution with streamed
+// loads and the change, in percent, with cached ones.  The caches are flushed
+// between the settings and warmed by each setting itself (settings that
+// alternate without it find the input where the other one left it).
+
+namespace {
+
+constexpr uint64_t kMiB = 1ull << 20;
+
+}  // namespace
 
 bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes) {
-    // Between 12 MiB and `top`, inputs that other buffers' executions have
-    // pushed out of the L2s load faster streamed (from the Infinity Cache).
-    // Measured on gfx950, us per execution, streamed / cached, three input /
-    // output pairs in turn:
-    // N = 128 14 MiB 5.32 / 5.66, 18 MiB 6.19 / 6.50, 26 MiB 11.2 / 8.8; 256
-    // 18 MiB 6.58 / 7.21, 24 MiB 8.21 / 8.67, 26 MiB 9.9 / 9.2; 512 18 MiB
-    // 6.97 / 7.43, 22 MiB 7.70 / 8.27, 30 MiB 11.1 / 10.5; 2048 22 MiB 8.55 /
-    // 8.90, 30 MiB 10.43 / 10.67, 34 MiB 12.4 / 11.7; 4096 18 MiB 7.97 / 8.37,
-    // 26 MiB 9.98 / 9.70, 32 MiB 10.90 / 11.26, 34 MiB 15.0 / 12.9; 8 and 10
-    // MiB 2 .. 15 % faster cached, 1024 (two transforms per workgroup) within
-    // 2 % or faster cached at all of these but 28 MiB (10.1 / 10.4), N <= 64
-    // 6 .. 20 % faster cached.  One pair again and again, its input partly in
-    // the L2 that reads it, gains 3 .. 17 % cached here too; buffers in turn
-    // and inputs written elsewhere are the case the rule serves.
-    const uint64_t top = log_n < 7 || log_n == 10 ? 0 : log_n <= 9 ? 24ull << 20 : 32ull << 20;
-    if (log_n <= 12 && bytes > 12ull << 20 && bytes <= top) return false;
-    return loads_cached(bytes, (log_n <= 12 ? 44ull : 16ull) << 20);
+    //                   one       turn      back      cold
+    //   N = 16   8 MiB  5.4 -20   5.5 -23   5.5 -7    5.5 +0
+    //            24 MiB 8.7 -32   8.9 -10   8.9 -3    8.8 +1
+    //            44 MiB 16.6 -13  17.0 -15  17.2 -1   17.3 +1
+    //            48 MiB 17.8 -13  18.0 -14  18.5 +2   18.6 +1
+    //   N = 64   20 MiB 8.7 -39   9.0 -21   9.4 -11   9.6 +0
+    //            44 MiB 16.6 -13  17.3 -15  17.3 -3   17.5 +1
+    //   N = 256  12 MiB 4.9 -13   5.2 -2    5.4 -2    5.5 +0
+    //            36 MiB 12.7 -7   13.5 -9   13.5 -5   13.9 +1
+    //            48 MiB 17.2 -11  18.0 -14  18.2 +2   18.3 +2
+    //   N = 1024 8 MiB  5.5 -24   5.7 -27   5.8 -10   5.8 -6
+    //            28 MiB 10.6 -19  10.9 -3   10.8 -3   10.7 -2
+    //            36 MiB 12.7 -6   13.2 -6   12.9 -1   12.9 +3
+    //   N = 4096 8 MiB  5.5 -14   5.7 -17   5.8 -2    5.8 +0
+    //            44 MiB 18.2 -14  18.8 -17  19.1 -4   19.1 +0
+    // 44 MiB is the size up to which callers there and back do not lose.
+    // Between 12 MiB and `top`, pairs in turn find little of their input in
+    // the L2s any more, and load as fast or faster streamed, from the Infinity
+    // Cache; the figures there are of processes that run one setting only, us,
+    // streamed / cached, one, turn, back, cold: N = 256 26 MiB 7.6 / 6.8, 9.0 /
+    // 9.4, 9.3 / 10.0, 9.5 / 10.3; 512 30 MiB 9.0 / 8.6, 10.5 / 10.3, 10.8 /
+    // 11.0, 11.2 / 12.2; 2048 36 MiB 11.1 / 12.5, 12.3 / 12.4, 12.7 / 13.0,
+    // 13.0 / 13.4; earlier, in turn: N = 128 14 MiB 5.32 / 5.66, 256 18 MiB
+    // 6.58 / 7.21, 512 22 MiB 7.70 / 8.27, 2048 22 MiB 8.55 / 8.90, 4096 32
+    // MiB 10.90 / 11.26, N <= 64 and 1024 faster cached or within 2 %.
+    //   N = 8192  12 MiB 9.3 -9    9.5 -5    9.6 +0    9.6 +0
+    //             24 MiB 12.4 +1   12.7 +6   13.3 +4   12.7 +1
+    //   N = 16384 16 MiB 13.9 -8   14.1 -6   14.2 -2   14.2 +0
+    //   N = 32768 16 MiB 21.9 -11  22.3 -8   22.5 -4   22.5 +0
+    uint64_t top = 0;
+    switch (log_n) {
+        case 7: top = 24 * kMiB; break;
+        case 8: top = 28 * kMiB; break;
+        case 9: top = 30 * kMiB; break;
+        case 11: top = 36 * kMiB; break;
+        case 12: top = 32 * kMiB; break;
+    }
+    if (bytes > 12 * kMiB && bytes <= top) return false;
+    return bytes <= (log_n <= 12 ? 44 : 16) * kMiB;
+}
+
+bool image_loads_cached(uint32_t log_points, uint64_t bytes) {
+    // One-pass images.
+    //                     one       turn      back      cold
+    //   16 x 16    24 MiB 8.8 -16   9.1 -4    9.2 -3    9.3 -0
+    //   32 x 64    8 MiB  6.8 -12   7.0 -14   7.1 -2    7.1 +0
+    //              12 MiB 7.6 -10   8.0 -0    8.2 +0    8.2 +0
+    //              16 MiB 8.7 -8    9.1 +4    9.3 +2    9.3 +0
+    //   128 x 128  16 MiB 15.3 -10  15.2 -5   15.4 -2   15.5 +0
+    //              24 MiB 16.1 -10  16.7 -4   16.9 +0   17.4 +1
+    // Of processes that run one setting only, streamed / cached: 64 x 64 24
+    // MiB 10.4 / 9.6, 11.8 / 12.2, 12.1 / 12.3, 12.6 / 12.8, 128 x 128 24 MiB
+    // 15.5 / 14.7, 16.4 / 16.5, 16.8 / 17.1, 17.4 / 17.8.
+    const uint64_t limit = log_points == 14 ? 20 : log_points >= FG_SMALL2D_HALVES_LOG ? 12 : 24;
+    return bytes <= limit * kMiB;
+}
+
+bool row_pass_loads_cached(uint64_t bytes) {
+    // Row passes of two-launch 2D plans.
+    //                        one       turn      back      cold
+    //   256 x 256     16 MiB 19.9 -7   15.8 -2   15.6 -1   16.2 +8
+    //                 24 MiB 25.1 -18  19.0 -2   18.9 -2   19.5 +4
+    //                 32 MiB 28.2 -21  24.5 -10  22.9 +4   25.9 +3
+    //                 40 MiB 32.4 -15  30.9 -10  29.9 +2   32.5 -3
+    //                 48 MiB 36.0 -12  35.7 -8   33.5 +6   37.2 -3
+    //   512 x 512     32 MiB 31.9 -22  27.2 -8   25.8 +2   28.0 +6
+    //                 40 MiB 35.0 -16  33.6 -11  31.6 +3   34.8 -2
+    //   1024 x 1024   24 MiB 28.8 -15  23.2 -3   23.2 -3   23.5 +3
+    //                 32 MiB 31.6 -17  26.9 -3   26.8 -0   27.2 +9
+    //                 40 MiB 40.7 -14  38.6 -9   37.0 +2   39.7 +1
+    //   128 x 512     32 MiB 31.8 -19  27.3 -6   26.1 +2   27.3 +11
+    //                 40 MiB 35.1 -17  32.9 -11  31.1 +4   34.6 -3
+    // Cold inputs lose most around 32 MiB, the size of the eight L2s, where the
+    // input takes the place of the rows that just fit them; the limit weighs
+    // them against the other three.
+    return bytes <= 40 * kMiB;
+}
+
+bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes) {
+    // First passes of 1D multi-pass plans, up to 56 MiB, 80 for 2^18 .. 2^20
+    // points, 32 where the last pass stores through the caches too (8-row
+    // tiles of 512 points).  In narrow forms up to 32 MiB (narrow_width), the
+    // pass's own tiles above:
+    //               one       turn      back      cold
+    //   2^16 16 MiB 21.1 -3   21.1 -2   21.2 -1   21.5 +6
+    //        32 MiB 29.0 -20  29.0 -20  29.2 -19  29.1 -17
+    //        48 MiB 38.8 -14  38.6 -14  39.0 -9   39.0 -10
+    //        56 MiB 43.2 -13  43.1 -13  43.1 +1   43.2 -0
+    //   2^17 24 MiB 23.9 -1   23.9 -1   24.2 -2   24.3 +7
+    //        28 MiB 25.3 -5   25.1 -4   26.0 +4   25.4 +10
+    //        32 MiB 27.7 -9   27.2 -8   26.5 +2   27.2 +11
+    //        40 MiB 32.2 -2   32.1 +5   31.8 +7   32.8 +9
+    //   2^18 16 MiB 19.3 -5   19.9 -4   19.8 -2   20.4 +6
+    //        32 MiB 27.4 -2   27.4 -2   27.5 +2   28.0 +12
+    //        64 MiB 48.8 -7   48.6 -6   48.2 -2   48.8 -2
+    //        80 MiB 60.5 -8   60.6 -1   62.2 -1   60.6 -1
+    //   2^20 32 MiB 31.8 -8   31.9 -8   30.8 +2   32.1 +10
+    //        64 MiB 51.8 -8   51.9 -7   52.6 -4   52.1 -4
+    //        80 MiB 68.8 -10  68.9 +1   70.1 +1   69.0 +1
+    //   2^22 32 MiB 41.1 -11  41.2 -11  41.7 -10  41.2 -7
+    // The narrow forms load through the caches whatever the plan's input (up
+    // to 32 MiB; as measured here they could stream).  Cold inputs of 28 to 32
+    // MiB lose 6 to 7 % at 2^17 against the plan without narrow forms (26.6 ->
+    // 28.2, 27.1 -> 29.1), where the other kinds gain 2 to 11.
+    const uint64_t limit = last_g < 16 ? 32 : log_n >= 18 && log_n <= 20 ? 80 : 56;
+    return bytes <= limit * kMiB;
 }
 
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
@@ -637,8 +707,7 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         t.ocs = 1;
         t.oes = N / L;
         p->add_tile(mod, log_l, g, true, t, (uint64_t)t.t0n * t.t1n, Buf::Work, Buf::Out, p->policy(P - 1, P));
-        const uint64_t cached_limit = (g < 16 ? 32ull : log_n >= 18 && log_n <= 20 ? 80ull : 56ull) << 20;
-        p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * N * batch, cached_limit);
+        p->load_cached_ = p->cached_ && p->chunks() == 1 && column_pass_loads_cached(log_n, g, 8ull * N * batch);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -689,7 +758,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = s.name;
         p->split_fn_ = HipBackend::get_kernel(mod, (s.name + "_split").c_str());
         p->pw_ = Pointwise(mod);
-        p->load_cached_ = batch <= (1u << 24) && loads_cached(8ull * RC * batch, 24ull << 20);
+        p->load_cached_ = batch <= (1u << 24) && image_loads_cached(log_rows + log_cols, 8ull * RC * batch);
         p->fit_launches();
         return p;
     }
@@ -702,7 +771,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
     // 256 324 -> 315, 1024 x 2048 378 -> 350, 32 x 1024 336 -> 314), 128 x
     // 2048 / 4096 and 512 x 4096 0.6 .. 1.3 % slower.
     p->choose_chunk(false);
-    p->load_cached_ = p->cached_ && p->chunks() == 1 && loads_cached(8ull * RC * batch, 40ull << 20);
+    p->load_cached_ = p->cached_ && p->chunks() == 1 && row_pass_loads_cached(8ull * RC * batch);
     if (split) p->work_ = dev.alloc<Cf32>(RC * p->chunk_);
     // Row pass (the reference's K1 row FFT, py lib.rs:325-336): R rows of C per image.
     p->add_stockham(mod, log_cols, R, Buf::In, split ? Buf::Work : Buf::Out, p->policy(0, npass));

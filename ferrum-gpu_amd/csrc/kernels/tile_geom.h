@@ -16,7 +16,7 @@ namespace fg {
 #define FG_PASS_CONJ (FG_PASS_CONJ_IN | FG_PASS_CONJ_SCALE_OUT)
 /* Kernels that stream their input in: load it through the caches instead (a
  * plan's first pass over an input small enough to stay in the Infinity
- * Cache; loads_cached in fft_plan.cpp). */
+ * Cache; *_loads_cached in fft_plan.cpp). */
 #define FG_PASS_LOAD_CACHED 4u
 /* Halves tile passes: flags >> FG_PASS_WIDTH_SHIFT is the columns per
  * workgroup of a launch in the kernel's narrow form (fft_tile_halves_pass),

@@ -1,4 +1,4 @@
-"""First passes that load their input through the caches (loads_cached,
+"""First passes that load their input through the caches (*_loads_cached,
 ferrum-gpu_amd/csrc/fft_plan.cpp): a batch below the limit gives the bits of
 the same transforms at the head of a batch above it, in both layouts, and
 agrees with numpy in double precision; ragged last workgroups included."""

@@ -1,0 +1,81 @@
+"""Dispatch rules of the plans (ferrum-gpu_amd/csrc/fft_plan.cpp), from the code
+itself: the file is compiled with g++ beside a small driver and the rules are
+asked at their edges.  What the rules choose changes no bits, so the GPU
+tests that compare results cannot see it."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "ferrum-gpu_amd", "csrc")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+MIB = 1 << 20
+
+# one rule per line: name, arguments, result
+PROGRAM = r"""
+#include <stdio.h>
+#include <string.h>
+#include "fft_plan.hpp"
+int main() {
+    char name[32];
+    unsigned long long a, b, c, d;
+    while (scanf("%31s %llu %llu %llu %llu", name, &a, &b, &c, &d) == 5) {
+        unsigned long long r = 0;
+        if (!strcmp(name, "single")) r = fg::single_pass_loads_cached(a, b);
+        else if (!strcmp(name, "image")) r = fg::image_loads_cached(a, b);
+        else if (!strcmp(name, "rows")) r = fg::row_pass_loads_cached(a);
+        else if (!strcmp(name, "columns")) r = fg::column_pass_loads_cached(a, b, c);
+        else return 1;
+        printf("%llu\n", r);
+    }
+    return 0;
+}
+"""
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None or not os.path.isdir(os.path.join(ROCM, "include", "hip")),
+                                reason="needs g++ and the ROCm headers")
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    src, exe = d / "rules.cpp", d / "rules"
+    src.write_text(PROGRAM)
+    # the rules call nothing outside their file, so the rest stays unresolved
+    subprocess.run(["g++", "-O0", "-std=c++17", "-D__HIP_PLATFORM_AMD__", f"-I{CSRC}", f"-I{os.path.join(ROOT, 'include')}",
+                    f"-I{os.path.join(ROCM, 'include')}", str(src), os.path.join(CSRC, "fft_plan.cpp"), "-o", str(exe),
+                    "-Wl,--unresolved-symbols=ignore-all"], check=True, capture_output=True, text=True, timeout=180)
+
+    def run(calls):
+        text = "".join(" ".join(str(v) for v in (list(c) + [0, 0, 0, 0])[:5]) + "\n" for c in calls)
+        out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True, timeout=60).stdout.split()
+        assert len(out) == len(calls)
+        return [int(v) for v in out]
+
+    return run
+
+
+def _edges(ask, rule, ranges):
+    """ranges: arguments -> (above, up to) in bytes, the inputs that load
+    through the caches."""
+    for args, (above, upto) in ranges.items():
+        sizes = [above, above + 8, upto, upto + 8] if above else [8, upto, upto + 8]
+        want = [0, 1, 1, 0] if above else [1, 1, 0]
+        assert ask([(rule, *args, s) for s in sizes]) == want, (rule, args)
+
+
+def test_first_passes_that_load_through_the_caches(ask):
+    for n, upto in [(n, 44) for n in (2, 3, 4, 5, 6, 10)] + [(13, 16), (14, 16), (15, 16)]:
+        _edges(ask, "single", {(n,): (0, upto * MIB)})
+    for n, top in ((7, 24), (8, 28), (9, 30), (11, 36), (12, 32)):  # streamed between 12 MiB and top
+        _edges(ask, "single", {(n,): (0, 12 * MIB)})
+        _edges(ask, "single", {(n,): (top * MIB, 44 * MIB)})
+    _edges(ask, "image", {(p,): (0, 24 * MIB) for p in (8, 9, 10)})
+    _edges(ask, "image", {(p,): (0, 12 * MIB) for p in (11, 12, 13)})
+    _edges(ask, "image", {(14,): (0, 20 * MIB)})
+    _edges(ask, "rows", {(): (0, 40 * MIB)})
+    _edges(ask, "columns", {(16, 32): (0, 56 * MIB), (17, 8): (0, 32 * MIB), (17, 16): (0, 56 * MIB), (18, 16): (0, 80 * MIB),
+                            (20, 16): (0, 80 * MIB), (21, 16): (0, 56 * MIB), (24, 32): (0, 56 * MIB)})
