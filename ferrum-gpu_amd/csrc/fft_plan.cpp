@@ -265,9 +265,47 @@ namespace {
 
 constexpr uint64_t kMiB = 1ull << 20;
 
+// Split layout: two f32 arrays, so a wave's access covers half the bytes of an
+// interleaved one, and streamed accesses that small cost more.
+bool split_single_pass_loads_cached(uint32_t log_n, uint64_t bytes) {
+    // 64 .. 256 points (4 to 16 lanes per transform) load through the caches
+    // at every size, 512 .. 4096 up to 64 MiB:
+    //                    one       turn      back      cold
+    //   N = 4     28 MiB 10.5 -38  10.8 -15  11.0 -8   11.0 +3
+    //   N = 16    44 MiB 15.6 -6   16.7 -12  16.9 +1   16.8 +3
+    //             64 MiB 22.7 -12  23.6 -16  23.4 +2   23.7 +2
+    //   N = 64    20 MiB 10.3 -47  10.4 -28  10.5 -17  10.6 -8
+    //             64 MiB 28.4 -22  27.9 -21  27.8 -7   27.9 -6
+    //             512 MiB 208 -14            205 -12
+    //   N = 128   16 MiB 7.0 -22   7.3 -2    7.4 +1    7.5 +4
+    //             512 MiB 208 -8             202 -9
+    //   N = 256   64 MiB 29.5 -15  29.1 -15  29.1 -11  29.4 -10
+    //             512 MiB 221 -9             212 -9
+    //   N = 512   20 MiB 7.2 -21   7.8 -3    7.8 -1    7.9 +1
+    //             64 MiB 23.1 -12  23.3 -14  23.2 +2   23.3 +2
+    //             96 MiB 33.5 -13  33.5 +5   33.6 +6   33.7 +5
+    //   N = 1024  16 MiB 6.3 -13   7.0 +3    7.2 +1    7.2 +0
+    //             64 MiB 24.2 -15  24.3 -15  24.2 +2   24.5 +2
+    //             96 MiB 34.9 -15  35.4 +6   35.0 +7   35.5 +6
+    //   N = 4096  64 MiB 25.4 -15  25.7 -16  25.7 +1   26.1 +2
+    //             96 MiB 35.7 -13  36.2 +8   36.5 +8   36.8 +7
+    //   N = 8192  24 MiB 12.6 -20  13.1 -2   13.4 -1   13.3 +2
+    //             32 MiB 13.9 -12  14.3 +0   14.6 +3   14.6 +6
+    //   N = 16384 24 MiB 14.2 -13  14.5 -1   14.7 +0   14.8 +2
+    //             64 MiB 24.5 +2   25.2 -0   25.2 +4   25.3 +4
+    //             512 MiB 200 +1             187 +7
+    //   N = 32768 32 MiB 23.4 -11  23.7 -2   24.0 -0   24.1 +2
+    // (N = 1024 16 MiB, of processes that run one setting only, in turn: 6.62
+    // streamed, 7.05 cached.)
+    if (log_n >= 6 && log_n <= 8) return true;
+    if (log_n == 10 && bytes > 12 * kMiB && bytes <= 20 * kMiB) return false;
+    return bytes <= (log_n < 6 ? 44 : log_n <= 12 ? 64 : log_n <= 14 ? 24 : 32) * kMiB;
+}
+
 }  // namespace
 
-bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes) {
+bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes, bool split) {
+    if (split) return split_single_pass_loads_cached(log_n, bytes);
     //                   one       turn      back      cold
     //   N = 16   8 MiB  5.4 -20   5.5 -23   5.5 -7    5.5 +0
     //            24 MiB 8.7 -32   8.9 -10   8.9 -3    8.8 +1
@@ -321,6 +359,10 @@ bool image_loads_cached(uint32_t log_points, uint64_t bytes) {
     // Of processes that run one setting only, streamed / cached: 64 x 64 24
     // MiB 10.4 / 9.6, 11.8 / 12.2, 12.1 / 12.3, 12.6 / 12.8, 128 x 128 24 MiB
     // 15.5 / 14.7, 16.4 / 16.5, 16.8 / 17.1, 17.4 / 17.8.
+    // Split layout: 16 x 16 24 MiB 9.0 -17, 9.7 -4, 9.8 -2, 9.7 +3, 32 MiB 11.6
+    // -17, 11.9 -6, 11.9 +4, 12.1 +11; 32 x 64 16 MiB 9.0 -9, 9.6 +5, 9.9 +2,
+    // 9.9 +0, 48 MiB 17.4 +5, 18.0 -3, 17.9 +6, 17.9 +6; 128 x 128 16 MiB 14.2
+    // -8, 14.3 -6, 14.5 -1, 14.4 +2, 32 MiB 18.2 -11, 18.7 -0, 18.9 +1, 18.9 +3.
     const uint64_t limit = log_points == 14 ? 20 : log_points >= FG_SMALL2D_HALVES_LOG ? 12 : 24;
     return bytes <= limit * kMiB;
 }
@@ -342,11 +384,14 @@ bool row_pass_loads_cached(uint64_t bytes) {
     //                 40 MiB 35.1 -17  32.9 -11  31.1 +4   34.6 -3
     // Cold inputs lose most around 32 MiB, the size of the eight L2s, where the
     // input takes the place of the rows that just fit them; the limit weighs
-    // them against the other three.
+    // them against the other three.  Split layout: 256 x 256 32 MiB 25.2 -11,
+    // 25.2 -11, 25.0 -3, 25.4 +12, 40 MiB 32.0 -18, 32.1 -17, 32.4 -8, 32.4 -6;
+    // 512 x 512 32 MiB 27.9 -6, 28.5 -7, 28.2 -2, 29.6 +1; 128 x 512 32 MiB 29.4
+    // -19, 29.3 -18, 29.2 -15, 28.9 -12.
     return bytes <= 40 * kMiB;
 }
 
-bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes) {
+bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes, bool split) {
     // First passes of 1D multi-pass plans, up to 56 MiB, 80 for 2^18 .. 2^20
     // points, 32 where the last pass stores through the caches too (8-row
     // tiles of 512 points).  In narrow forms up to 32 MiB (narrow_width), the
@@ -372,8 +417,39 @@ bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes) {
     // to 32 MiB; as measured here they could stream).  Cold inputs of 28 to 32
     // MiB lose 6 to 7 % at 2^17 against the plan without narrow forms (26.6 ->
     // 28.2, 27.1 -> 29.1), where the other kinds gain 2 to 11.
+    // Split layout, in the pass's own tiles above split_narrow_limit, up to 56
+    // MiB, 80 for 2^19 and 2^20 points, 32 for 8-row last tiles:
+    //   2^16 32 MiB 26.9 -6   26.8 -6   26.4 +1   27.2 +11
+    //        48 MiB 37.5 -10  38.2 -12  38.4 -3   38.3 -5
+    //   2^17 28 MiB 27.5 -5   27.5 -5   27.7 -2   27.9 +6
+    //        40 MiB 34.1 -3   34.3 +4   34.4 +8   34.9 +15
+    //   2^18 32 MiB 30.6 -4   30.5 -4   30.5 +0   31.2 +8
+    //        56 MiB 51.6 -14  51.9 -11  54.2 +0   52.3 +3
+    //        64 MiB 55.9 -9   54.1 -4   56.9 +3   54.1 +7
+    //   2^19 32 MiB 36.0 -14  35.9 -13  35.4 -7   36.4 -1
+    //        64 MiB 63.5 -22  63.0 -11  65.0 -1   63.4 +0
+    //   2^20 32 MiB 35.9 -9   35.9 -9   35.7 -3   36.6 +5
+    //        64 MiB 63.5 -17  62.5 -11  64.7 +2   62.8 +4
+    //        80 MiB 86.0 -20  85.6 -2   86.8 -1   85.5 -2
+    if (split) return bytes <= (last_g < 16 ? 32 : log_n >= 19 && log_n <= 20 ? 80 : 56) * kMiB;
     const uint64_t limit = last_g < 16 ? 32 : log_n >= 18 && log_n <= 20 ? 80 : 56;
     return bytes <= limit * kMiB;
+}
+
+uint64_t split_narrow_limit(uint32_t log_l) {
+    // A narrow form reads pieces of 4 W bytes of each of the two arrays, which
+    // the L2s join only while the launch's input and output leave them room:
+    // above, the pass's own tiles (whole lines of 32 columns at 256 points) are
+    // faster.  Loads through the caches, us per execution, narrow / own, one,
+    // turn, back, cold: 2^16 24 MiB 21.8 / 22.3, 21.9 / 22.4, 22.2 / 22.5, 25.9
+    // / 25.4, 28 MiB 23.7 / 24.0, 23.6 / 23.9, 27.2 / 25.3, 32.2 / 28.0, 32 MiB
+    // 24.3 / 25.2, 24.2 / 25.1, 28.5 / 26.5, 34.6 / 30.3; 2^18 32 MiB 29.0 /
+    // 29.3, 28.7 / 29.4, 32.5 / 30.5, 37.8 / 33.6; 2^19 24 MiB 27.8 / 29.2,
+    // 28.0 / 29.0, 28.3 / 29.9, 37.0 / 32.7, 28 MiB 31.0 / 29.0, 31.2 / 29.2,
+    // 35.7 / 31.0, 42.5 / 34.3; 2^20 16 MiB 24.8 / 27.5, 24.8 / 27.8, 25.3 /
+    // 27.9, 27.9 / 30.6, 24 MiB 29.9 / 28.8, 29.9 / 29.1, 30.6 / 29.5, 40.7 /
+    // 33.9, 32 MiB 32.4 / 32.4, 32.9 / 32.5, 37.9 / 34.5, 44.6 / 38.7.
+    return (log_l == 10 ? 16 : 24) * kMiB;
 }
 
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
@@ -637,7 +713,8 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = p->steps_[0].name;
         p->split_fn_ = HipBackend::get_kernel(mod, (p->main_kernel_ + "_split").c_str());
         p->pw_ = Pointwise(mod);
-        p->load_cached_ = batch <= (1u << 24) && single_pass_loads_cached(log_n, (8ull * batch) << log_n);
+        for (const bool split : {false, true})
+            p->load_cached_[split] = batch <= (1u << 24) && single_pass_loads_cached(log_n, (8ull * batch) << log_n, split);
         p->fit_launches();
         return p;
     }
@@ -707,7 +784,9 @@ std::unique_ptr<FftPlan> FftPlan::make_1d(HipDevice& dev, const HipBackend::Modu
         t.ocs = 1;
         t.oes = N / L;
         p->add_tile(mod, log_l, g, true, t, (uint64_t)t.t0n * t.t1n, Buf::Work, Buf::Out, p->policy(P - 1, P));
-        p->load_cached_ = p->cached_ && p->chunks() == 1 && column_pass_loads_cached(log_n, g, 8ull * N * batch);
+        for (const bool split : {false, true})
+            p->load_cached_[split] =
+                p->cached_ && p->chunks() == 1 && column_pass_loads_cached(log_n, g, 8ull * N * batch, split);
         if (two) {
             // Two chunks in flight, one per stream: their passes overlap, so
             // one chunk's transform phases fill the other's memory phases.
@@ -758,7 +837,8 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
         p->main_kernel_ = s.name;
         p->split_fn_ = HipBackend::get_kernel(mod, (s.name + "_split").c_str());
         p->pw_ = Pointwise(mod);
-        p->load_cached_ = batch <= (1u << 24) && image_loads_cached(log_rows + log_cols, 8ull * RC * batch);
+        p->load_cached_[0] = p->load_cached_[1] =
+            batch <= (1u << 24) && image_loads_cached(log_rows + log_cols, 8ull * RC * batch);
         p->fit_launches();
         return p;
     }
@@ -771,7 +851,7 @@ std::unique_ptr<FftPlan> FftPlan::make_2d(HipDevice& dev, const HipBackend::Modu
     // 256 324 -> 315, 1024 x 2048 378 -> 350, 32 x 1024 336 -> 314), 128 x
     // 2048 / 4096 and 512 x 4096 0.6 .. 1.3 % slower.
     p->choose_chunk(false);
-    p->load_cached_ = p->cached_ && p->chunks() == 1 && row_pass_loads_cached(8ull * RC * batch);
+    p->load_cached_[0] = p->load_cached_[1] = p->cached_ && p->chunks() == 1 && row_pass_loads_cached(8ull * RC * batch);
     if (split) p->work_ = dev.alloc<Cf32>(RC * p->chunk_);
     // Row pass (the reference's K1 row FFT, py lib.rs:325-336): R rows of C per image.
     p->add_stockham(mod, log_cols, R, Buf::In, split ? Buf::Work : Buf::Out, p->policy(0, npass));
@@ -979,7 +1059,7 @@ void FftPlan::run(const std::vector<Step>& steps, const Arrays& a, Direction dir
             uint32_t flags = 0;
             if (inverse && i == 0) flags |= FG_PASS_CONJ_IN;
             if (inverse && i + 1 == steps.size()) flags |= FG_PASS_CONJ_SCALE_OUT;
-            if (i == 0 && load_cached_) flags |= FG_PASS_LOAD_CACHED;
+            if (i == 0 && load_cached_[split_in]) flags |= FG_PASS_LOAD_CACHED;
             void* args[9];
             size_t n = 0;
             // Input and output: one interleaved pointer each, or re and im.
@@ -1028,7 +1108,8 @@ void FftPlan::run(const std::vector<Step>& steps, const Arrays& a, Direction dir
                 // Columns that share a 128-byte line: 16, or 32 of an f32 array.
                 const uint32_t line = split_in || split_out ? 32 : 16;
                 uint32_t order = s.tile_order, order_unit = s.order_unit, w = s.width;
-                if (const uint32_t narrow = s.narrows && !two ? narrow_width(s.log_l, s.width, count, cu_count) : 0) {
+                const bool narrows = s.narrows && !two && !(split_in && 8 * unit * units > split_narrow_limit(s.log_l));
+                if (const uint32_t narrow = narrows ? narrow_width(s.log_l, s.width, count, cu_count) : 0) {
                     const uint32_t k = s.width / narrow;  // the geometry steps tiles by the width (add_tile)
                     w = narrow;
                     count *= k;
@@ -1082,7 +1163,7 @@ void FftPlan::split_one_launch(const void* in_re, const void* in_im, void* out_r
                                bool normalize, hipStream_t stream) const {
     const Step& s = steps_[0];  // the split twin has the same geometry and table
     uint32_t flags = dir == Direction::Inverse ? FG_PASS_CONJ : 0u;
-    if (load_cached_) flags |= FG_PASS_LOAD_CACHED;
+    if (load_cached_[1]) flags |= FG_PASS_LOAD_CACHED;
     float sc = scale_for(dir, normalize);
     const void* tw = s.tw;
     const void* twc = s.tw_cols;

@@ -230,7 +230,7 @@ private:
     size_t batch_;
     size_t chunk_;         // units per chunk (batch_ when not chunked)
     bool cached_ = false;  // intermediates kept cached (else every pass streams)
-    bool load_cached_ = false;  // the first pass loads its input through the caches (*_loads_cached)
+    bool load_cached_[2] = {false, false};  // [split layout]: the first pass loads its input through the caches (*_loads_cached)
     std::vector<Step> steps_;
     std::vector<Step> steps_in_place_;  // when not empty: the passes of in-place executions (in == out)
     std::vector<std::pair<uint32_t, Buffer<Cf32, HipBackend>>> stage_tables_;
@@ -283,11 +283,15 @@ bool use_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
 bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise);
 // Whether a plan whose whole input is `bytes` loads it through the caches: 1D
 // single-pass plans, one-pass 2D plans, the row pass of two-launch 2D plans,
-// the first pass of 1D multi-pass plans (last_g: rows per tile of the last).
-bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes);
+// the first pass of 1D multi-pass plans (last_g: rows per tile of the last);
+// split: from the split layout's two arrays.
+bool single_pass_loads_cached(uint32_t log_n, uint64_t bytes, bool split);
 bool image_loads_cached(uint32_t log_points, uint64_t bytes);
 bool row_pass_loads_cached(uint64_t bytes);
-bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes);
+bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes, bool split);
+// Bytes of a launch's split input up to which a first pass of 2^log_l points
+// may run in a narrow form.
+uint64_t split_narrow_limit(uint32_t log_l);
 // Columns per workgroup of a launch of `tiles` tiles of a pass (2^log_l points, g columns per tile) in its narrow form; 0: its own tiles.
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count);
 // Whether the column FFT of an image with 2^log_rows rows runs as two passes.

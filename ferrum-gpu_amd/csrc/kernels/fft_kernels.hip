@@ -461,13 +461,14 @@ FG_TILE_NARROW(9, 8, true, r)
 // instead of an interleaving and a deinterleaving pass around the plan (two
 // of its four or five passes over the array).  Tiles of fewer than 32 columns
 // move less than a 128-byte line of each array; the tiles of a line run on
-// one XCD (FG_TILE_ORDER_LINE_GROUPS).  They still stream the caller's
-// arrays: through the caches 16-column tiles displaced the intermediate
-// (cached / streamed, us per execution: 2^18 at 256 MiB 276 / 206, 2^20 at 64
-// MiB 68 / 53, 1024 x 1024 at 192 MiB 181 / 136; 512 x 512 at 48 MiB 40 /
-// 43).  Measured on gfx950 against the staged form, us: 2^18 x 16 63.8 ->
-// 28.1, 2^16 x 64 59.5 -> 24.2, 2^20 x 1 37.0 -> 18.6, 2^24 x 1 219 -> 136,
-// 512 x 512 x 3 25.8 -> 12.2, 256 x 256 x 200 138.7 -> 67.3.
+// one XCD (FG_TILE_ORDER_LINE_GROUPS).  First passes load the arrays through
+// the caches or streamed, and in narrow forms or their own tiles, by the split
+// layout's own limits (column_pass_loads_cached, split_narrow_limit in
+// fft_plan.cpp); last passes stream their stores from their own tiles of 16
+// columns and more, and store through the caches from narrow ones.  Measured
+// on gfx950 against the staged form, us: 2^18 x 16 63.8 -> 28.1, 2^16 x 64
+// 59.5 -> 24.2, 2^20 x 1 37.0 -> 18.6, 2^24 x 1 219 -> 136, 512 x 512 x 3 25.8
+// -> 12.2, 256 x 256 x 200 138.7 -> 67.3.
 #define FG_TILE_SPLIT_IN(LOGL, G)                                                                          \
     extern "C" __global__ __launch_bounds__(G * HalvesShape<LOGL>::T) __attribute__((amdgpu_waves_per_eu(4))) \
     void fg_tile_l##LOGL##_g##G##_h_si(const float* __restrict__ in_re, const float* __restrict__ in_im,       \

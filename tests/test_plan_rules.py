@@ -24,10 +24,11 @@ int main() {
     unsigned long long a, b, c, d;
     while (scanf("%31s %llu %llu %llu %llu", name, &a, &b, &c, &d) == 5) {
         unsigned long long r = 0;
-        if (!strcmp(name, "single")) r = fg::single_pass_loads_cached(a, b);
+        if (!strcmp(name, "single")) r = fg::single_pass_loads_cached(a, b, c);
         else if (!strcmp(name, "image")) r = fg::image_loads_cached(a, b);
         else if (!strcmp(name, "rows")) r = fg::row_pass_loads_cached(a);
-        else if (!strcmp(name, "columns")) r = fg::column_pass_loads_cached(a, b, c);
+        else if (!strcmp(name, "columns")) r = fg::column_pass_loads_cached(a, b, c, d);
+        else if (!strcmp(name, "split_narrow")) r = fg::split_narrow_limit(a);
         else return 1;
         printf("%llu\n", r);
     }
@@ -58,13 +59,13 @@ def ask(tmp_path_factory):
     return run
 
 
-def _edges(ask, rule, ranges):
+def _edges(ask, rule, ranges, *last):
     """ranges: arguments -> (above, up to) in bytes, the inputs that load
-    through the caches."""
+    through the caches; last: the rule's arguments after the size."""
     for args, (above, upto) in ranges.items():
         sizes = [above, above + 8, upto, upto + 8] if above else [8, upto, upto + 8]
         want = [0, 1, 1, 0] if above else [1, 1, 0]
-        assert ask([(rule, *args, s) for s in sizes]) == want, (rule, args)
+        assert ask([(rule, *args, s, *last) for s in sizes]) == want, (rule, args)
 
 
 def test_first_passes_that_load_through_the_caches(ask):
@@ -79,3 +80,14 @@ def test_first_passes_that_load_through_the_caches(ask):
     _edges(ask, "rows", {(): (0, 40 * MIB)})
     _edges(ask, "columns", {(16, 32): (0, 56 * MIB), (17, 8): (0, 32 * MIB), (17, 16): (0, 56 * MIB), (18, 16): (0, 80 * MIB),
                             (20, 16): (0, 80 * MIB), (21, 16): (0, 56 * MIB), (24, 32): (0, 56 * MIB)})
+
+
+def test_split_inputs_have_limits_of_their_own(ask):
+    limits = {2: 44, 3: 44, 4: 44, 5: 44, 9: 64, 11: 64, 12: 64, 13: 24, 14: 24, 15: 32}
+    _edges(ask, "single", {(n,): (0, limits[n] * MIB) for n in limits}, 1)
+    _edges(ask, "single", {(10,): (0, 12 * MIB)}, 1)  # streamed up to 20 MiB
+    _edges(ask, "single", {(10,): (20 * MIB, 64 * MIB)}, 1)
+    assert all(ask([("single", n, s, 1) for n in (6, 7, 8) for s in (8, MIB, 4096 * MIB)]))  # no limit
+    _edges(ask, "columns", {(16, 32): (0, 56 * MIB), (17, 8): (0, 32 * MIB), (17, 16): (0, 56 * MIB), (18, 16): (0, 56 * MIB),
+                            (19, 16): (0, 80 * MIB), (20, 16): (0, 80 * MIB), (21, 16): (0, 56 * MIB)}, 1)
+    assert ask([("split_narrow", log_l) for log_l in (7, 8, 9, 10)]) == [24 * MIB, 24 * MIB, 24 * MIB, 16 * MIB]
