@@ -525,9 +525,12 @@ size_t chunk_units_for(uint64_t unit_bytes, size_t batch, size_t limit, bool* ca
     return (size_t)std::min<uint64_t>(limit / unit_bytes, batch);
 }
 
-bool FftPlan::choose_chunk(bool two_in_flight) {
-    const size_t limit = chunk_limit_bytes();
-    const uint64_t unit = 8ull * elems();
+bool makes_two_chunks(uint64_t unit_bytes, size_t batch, size_t limit) {
+    bool cached = false;
+    return unit_bytes <= limit / 2 && chunk_units_for(unit_bytes, batch, limit / 2, &cached) < batch;
+}
+
+bool runs_two_chunks(uint64_t unit_bytes, size_t batch, size_t limit) {
     // Two chunks in flight from a batch of the limit up.  Below it one chunk
     // on one stream is faster: the second stream's fork and join cost about 15
     // us, and the last chunk is a remainder.  Measured on gfx950 under the
@@ -537,13 +540,17 @@ bool FftPlan::choose_chunk(bool two_in_flight) {
     // / 182.3, 2^22 224 MiB 224.7 / 215.8.  From 512 MiB (two or more chunks
     // of 256 MiB on one stream) it loses: 2^16 323.3 / 344.5, 2^24 480.8 /
     // 515.2.
-    const uint64_t all = unit > SIZE_MAX / batch_ ? SIZE_MAX : unit * batch_;
-    if (two_in_flight && all >= limit && unit <= limit / 2) {
-        chunk_ = chunk_units_for(unit, batch_, limit / 2, &cached_);
-        if (chunks() > 1) return true;
-    }
-    chunk_ = chunk_units_for(unit, batch_, limit, &cached_);
-    return false;
+    const uint64_t all = unit_bytes > SIZE_MAX / batch ? SIZE_MAX : unit_bytes * batch;
+    return all >= limit && makes_two_chunks(unit_bytes, batch, limit);
+}
+
+bool FftPlan::choose_chunk(bool two_in_flight) {
+    const size_t limit = chunk_limit_bytes();
+    const uint64_t unit = 8ull * elems();
+    takes_two_ = two_in_flight && makes_two_chunks(unit, batch_, limit);
+    const bool two = two_in_flight && runs_two_chunks(unit, batch_, limit);
+    chunk_ = chunk_units_for(unit, batch_, two ? limit / 2 : limit, &cached_);
+    return two;
 }
 
 const char* FftPlan::policy(size_t i, size_t n) const {
@@ -679,7 +686,8 @@ FftPlan::ChunkStream::~ChunkStream() {
 
 void FftPlan::set_streams(int n) {
     if (n != 1 && n != 2) invalid("streams must be 1 or 2, got " + std::to_string(n));
-    if (n == 2 && !aux_) invalid("this plan runs on one stream (two-stream plans: multi-pass 1D of two or more chunks)");
+    if (n == 2 && !takes_two_)
+        invalid("this plan runs on one stream (2: multi-pass 1D plans whose batch exceeds half the chunk limit)");
     use_aux_ = n == 2;
 }
 

@@ -75,8 +75,11 @@ public:
     // workspace and events).
     int max_streams() const { return aux_ ? 2 : 1; }
     // Runs the plan's chunks on one stream (1) or, where max_streams() is 2,
-    // alternately on two (2, the default).  Same bits either way; executions
-    // must not be in flight while it changes.
+    // alternately on two (2, the default).  2 changes nothing on the other
+    // plans whose batch would make two chunks of half the limit, which run
+    // it as one chunk because that is faster (runs_two_chunks), and is refused
+    // elsewhere.  Same bits either way; executions must not be in flight
+    // while it changes.
     void set_streams(int n);
     // The stream a chunk's launches run on: 0 the caller's, 1 the device's
     // chunk stream (HipBackend::chunk_stream).
@@ -239,6 +242,7 @@ private:
     Buffer<Cf32, HipBackend> work2_;         // the odd chunks' workspace (two-stream 1D plans)
     std::unique_ptr<ChunkStream> aux_;       // two-stream plans: the odd chunks' stream
     bool use_aux_ = true;                    // set_streams
+    bool takes_two_ = false;                 // two chunks of half the limit hold the batch: set_streams(2) is taken
     std::string main_kernel_;
     HipBackend::KernelHandle split_fn_ = nullptr;  // single-pass plans: the split-layout twin
     Pointwise pw_;
@@ -305,6 +309,10 @@ void set_chunk_limit_bytes(size_t bytes);
 // Units per chunk for `unit_bytes` per transform (image), and whether the
 // chunk's intermediates are kept cached, under the given limit.
 size_t chunk_units_for(uint64_t unit_bytes, size_t batch, size_t limit, bool* cached);
+// Whether a batch makes two or more chunks of half the limit (multi-pass 1D
+// plans then take set_streams(2)), and whether it runs them two at a time.
+bool makes_two_chunks(uint64_t unit_bytes, size_t batch, size_t limit);
+bool runs_two_chunks(uint64_t unit_bytes, size_t batch, size_t limit);
 // Whether a single-pass plan of `count` transforms of 2^log_n points runs the
 // latency geometry (fg_fft_n<L>_lat) on a device with `cu_count` CUs.
 bool use_latency_geometry(uint32_t log_n, uint64_t count, int cu_count);

@@ -276,8 +276,9 @@ class _Plan:
 
     def set_streams(self, streams: int) -> None:
         """Run the chunks on one stream (1) or, for a plan created with
-        describe()["streams"] == 2, on two again (2); same bits either way.
-        No execution of the plan may be in flight."""
+        describe()["streams"] == 2, on two again (2; accepted without effect
+        by multi-pass 1D plans of between half the chunk limit and the limit,
+        which run one chunk); same bits either way.  No execution of the plan may be in flight."""
         _n.check(_n.lib.fg_fft_plan_set_streams(self._p, int(streams)))
 
     def describe(self) -> dict:

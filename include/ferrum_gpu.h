@@ -222,8 +222,8 @@ FG_API int fg_fft_get_chunk_bytes(size_t *bytes);
  * are kept cached (1) or every pass streams (0). */
 FG_API int fg_fft_plan_chunking(fg_fft_plan_t plan, int *passes, size_t *units_per_chunk, int *chunks,
                                 int *cached);
-/* Streams an execution runs on: 1, or 2 for multi-pass 1D plans of two or
- * more chunks, which run the odd chunks (launches passes*c .. passes*c +
+/* Streams an execution runs on: 1, or 2 for multi-pass 1D plans whose batch
+ * takes the chunk limit or more, in two or more chunks, which run the odd chunks (launches passes*c .. passes*c +
  * passes - 1 of chunk c) with a second workspace on the device's chunk
  * stream (one per device, shared by every two-stream plan on it), forked
  * from the caller's stream when the execution starts and joined back to it
@@ -236,7 +236,10 @@ FG_API int fg_fft_plan_chunking(fg_fft_plan_t plan, int *passes, size_t *units_p
 FG_API int fg_fft_plan_streams(fg_fft_plan_t plan, int *streams);
 /* Runs a plan's chunks on one stream (streams = 1) or, for a plan that
  * fg_fft_plan_streams reported at 2 when it was created, on two again
- * (streams = 2; FG_ERR_INVALID_ARGUMENT for other plans or values).  Same
+ * (streams = 2).  Multi-pass 1D plans whose batch exceeds half the chunk limit
+ * and stays below it run one chunk on one stream and accept 2 without
+ * effect; FG_ERR_INVALID_ARGUMENT for 2 on other plans and for other
+ * values.  Same
  * results bit for bit either way; no execution of the plan may be in flight
  * while it changes.  For callers whose own streams already occupy the
  * hardware queues, and for timing each pass on its own.  No counterpart in

@@ -316,3 +316,35 @@ def test_set_streams_one_and_back_same_bits(gpu_device, chunk_limit):
         p.destroy()
     a.free()
     b.free()
+
+
+def test_set_streams_two_on_a_plan_of_one_chunk(gpu_device, chunk_limit):
+    # a batch between half the chunk limit and the limit runs as one chunk on
+    # one stream; set_streams(2) is accepted there without effect, and refused
+    # for a batch of half the limit
+    import ferrum_gpu
+    from ferrum_gpu.hip import DeviceBuffer
+
+    log_n = 17
+    n = 1 << log_n
+    chunk_limit(4 * n * 8)
+    plan, half = ferrum_gpu.fft.Plan1D(log_n, 3, gpu_device), ferrum_gpu.fft.Plan1D(log_n, 2, gpu_device)
+    print(f"[case] set_streams(2) on one chunk {plan.describe()}", flush=True)
+    x = normal_c64(np.random.default_rng(92), 3 * n)
+    a, b = DeviceBuffer(gpu_device, plan.nbytes), DeviceBuffer(gpu_device, plan.nbytes)
+    a.copy_from_host(x)
+    outs = []
+    for streams in (2, 1, 2):
+        plan.set_streams(streams)
+        d = plan.describe()
+        assert d["streams"] == 1 and d["chunks"] == 1
+        plan.execute(a, b, "forward")
+        gpu_device.sync()
+        outs.append(b.copy_to_host(np.empty_like(x)))
+    assert all(np.array_equal(o.view(np.uint32), outs[0].view(np.uint32)) for o in outs)
+    assert _lanes(outs[0], x, log_n, 3) <= TOL
+    with pytest.raises(Exception):
+        half.set_streams(2)
+    half.set_streams(1)
+    for p in (plan, half):
+        p.destroy()

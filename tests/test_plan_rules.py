@@ -29,6 +29,8 @@ int main() {
         else if (!strcmp(name, "rows")) r = fg::row_pass_loads_cached(a);
         else if (!strcmp(name, "columns")) r = fg::column_pass_loads_cached(a, b, c, d);
         else if (!strcmp(name, "split_narrow")) r = fg::split_narrow_limit(a);
+        else if (!strcmp(name, "makes_two")) r = fg::makes_two_chunks(a, b, c);
+        else if (!strcmp(name, "runs_two")) r = fg::runs_two_chunks(a, b, c);
         else return 1;
         printf("%llu\n", r);
     }
@@ -91,3 +93,13 @@ def test_split_inputs_have_limits_of_their_own(ask):
     _edges(ask, "columns", {(16, 32): (0, 56 * MIB), (17, 8): (0, 32 * MIB), (17, 16): (0, 56 * MIB), (18, 16): (0, 56 * MIB),
                             (19, 16): (0, 80 * MIB), (20, 16): (0, 80 * MIB), (21, 16): (0, 56 * MIB)}, 1)
     assert ask([("split_narrow", log_l) for log_l in (7, 8, 9, 10)]) == [24 * MIB, 24 * MIB, 24 * MIB, 16 * MIB]
+
+
+def test_two_chunks_run_at_once_from_a_batch_of_the_limit(ask):
+    # unit, batch, limit -> (takes set_streams(2), runs two chunks at a time)
+    cases = {(MIB, 128, 256 * MIB): (0, 0), (MIB, 129, 256 * MIB): (1, 0), (MIB, 255, 256 * MIB): (1, 0),
+             (MIB, 256, 256 * MIB): (1, 1), (128 * MIB, 1, 256 * MIB): (0, 0), (128 * MIB, 2, 256 * MIB): (1, 1),
+             (3 * MIB, 5, 4 * MIB): (0, 0), (MIB, 7, 0): (0, 0), (8 * MIB, 7, 4 * MIB): (0, 0),
+             (1 << 40, (1 << 40) - 1, 2**63): (1, 1)}  # unit * batch beyond 2^64
+    assert ask([("makes_two", *c) for c in cases]) == [m for m, _ in cases.values()]
+    assert ask([("runs_two", *c) for c in cases]) == [r for _, r in cases.values()]
