@@ -28,23 +28,28 @@ def _run(dev, plan, x, direction, normalize, in_place=False):
 
 
 # (log_rows or 0, log_n, batches, a batch whose launches keep their own tiles):
-# 1D 2^16: 8 tiles per transform, 4 columns to 4 transforms, 8 to 32, 16 to
-# 128; 2^18: 32 / 16; 2^19, 2^20: 64 / 32 and 64 / 64.  2D: C / width tiles.
+# on 256 CUs both sides of every width's limit (narrow_width; each limit is
+# asked of the rule itself in test_plan_rules.py).  Transforms or images up to
+# which a launch takes 4 / 8 / 16 columns: 2^16 4 / 32 / 64; 2^17 first pass 2 /
+# 16 / 32, last 4; 2^18 first 1 / 8 / 16, last 4 / 16; 2^19 first 1 / 8, last 2 / 8;
+# 2^20 1 / 4; 2^21, 2^22 - / - / 1; 128 rows x 1024 - / 8 / 16; 256 x 256 4 / 32 /
+# 64; 512 x 512 2 / 16; 1024 x 1024 1 / 4; 1024 x 256 4 / 16; 2048 x 16 64; 4096 x
+# 64 16.
 SHAPES = [
-    (0, 16, (1, 4, 5, 32, 33, 128), 131),
-    (0, 17, (1, 4, 5, 17, 39), 70),
-    (0, 18, (1, 2, 3, 9, 17), 34),
-    (0, 19, (1, 5), 18),
-    (0, 20, (1, 2, 5), 9),
+    (0, 16, (1, 4, 5, 32, 33, 64, 65), 131),
+    (0, 17, (1, 2, 3, 4, 5, 16, 17, 32, 33), 70),
+    (0, 18, (1, 2, 4, 5, 8, 9, 16, 17), 34),
+    (0, 19, (1, 2, 3, 8, 9), 18),
+    (0, 20, (1, 2, 4, 5), 9),
     (0, 21, (1, 2), 5),
-    (0, 22, (1,), 3),
-    (7, 10, (1, 8, 9, 17), 70),
-    (8, 8, (1, 8, 9, 33, 65), 130),
-    (9, 9, (1, 2, 3, 17), 34),
-    (10, 10, (1, 2, 5), 9),
-    (10, 8, (1, 4, 17), 33),
-    (11, 4, (1, 64), 129),
-    (12, 6, (1, 8), 17),
+    (0, 22, (1, 2), 3),
+    (7, 10, (1, 8, 9, 16, 17), 70),
+    (8, 8, (1, 4, 5, 32, 33, 64, 65), 130),
+    (9, 9, (1, 2, 3, 16, 17), 34),
+    (10, 10, (1, 2, 4, 5), 9),
+    (10, 8, (1, 4, 5, 16, 17), 33),
+    (11, 4, (1, 64, 65), 129),
+    (12, 6, (1, 16, 17), 33),
 ]
 
 

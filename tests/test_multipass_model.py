@@ -59,8 +59,8 @@ def split_1d(log_n):
 def tile_geometry_1d(log_n, batch, cached=True, streams=1):
     """Per-pass geometry dicts (TileGeom), built as FftPlan::make_1d builds them;
     ``cached``: the plan is chunked, so passes after the first read the caches;
-    ``chunks``: how many chunks the batch takes (two or more: the last pass
-    takes at least 16 rows, for the plan's two chunks in flight)."""
+    ``streams``: 2 for two chunks in flight, whose last pass takes at least 16
+    rows (as one chunk of more than 40 MiB does)."""
     logs = split_1d(log_n)
     P = len(logs)
     N = 1 << log_n
@@ -133,15 +133,15 @@ def two_in_flight_shape(two_d, log_rows, log_cols=None):
 def choose_chunk(unit, batch, limit, two_in_flight):
     """FftPlan::choose_chunk (fft_plan.cpp): (units per chunk, cached, two chunks
     in flight).  The limit bounds the bytes in flight: chunks of limit / 2 for
-    shapes that run two at a time when a unit fits and the batch makes two or
-    more, else chunks of the limit; 0 or a unit above the limit: one
-    streaming chunk."""
+    shapes that run two at a time when a unit fits, the batch takes the limit
+    and makes two or more, else chunks of the limit; 0 or a unit above the
+    limit: one streaming chunk."""
     def units_for(lim):
         if lim == 0 or unit > lim:
             return batch, False
         return min(lim // unit, batch), True
 
-    if two_in_flight and unit <= limit // 2:
+    if two_in_flight and unit * batch >= limit and unit <= limit // 2:
         per, cached = units_for(limit // 2)
         if -(-batch // per) > 1:
             return per, cached, True
@@ -486,7 +486,11 @@ def test_chunk_choice_bounds_the_bytes_in_flight():
     assert choose_chunk(128 * MIB, 2, 256 * MIB, False) == (2, True, False)
     # a batch that fits half the limit: one chunk, one stream
     assert choose_chunk(MIB, 100, 256 * MIB, True) == (100, True, False)
-    # 512 MiB of 2D 256 x 256 images: 128 MiB chunks, two in flight
+    # between half the limit and the limit: one chunk, one stream
+    assert choose_chunk(MIB, 200, 256 * MIB, True) == (200, True, False)
+    # the limit: two chunks of half of it in flight
+    assert choose_chunk(MIB, 256, 256 * MIB, True) == (128, True, True)
+    # units of 512 KiB, 512 MiB of them: 128 MiB chunks, two in flight
     assert choose_chunk(512 * 1024, 1024, 256 * MIB, True) == (256, True, True)
     # a unit above half the limit: one chunk at a time of the whole limit
     assert choose_chunk(3 * MIB, 5, 4 * MIB, True) == (1, True, False)

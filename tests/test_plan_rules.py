@@ -31,6 +31,7 @@ int main() {
         else if (!strcmp(name, "split_narrow")) r = fg::split_narrow_limit(a);
         else if (!strcmp(name, "makes_two")) r = fg::makes_two_chunks(a, b, c);
         else if (!strcmp(name, "runs_two")) r = fg::runs_two_chunks(a, b, c);
+        else if (!strcmp(name, "narrow")) r = fg::narrow_width(a, b, c, d);
         else return 1;
         printf("%llu\n", r);
     }
@@ -103,3 +104,35 @@ def test_two_chunks_run_at_once_from_a_batch_of_the_limit(ask):
              (1 << 40, (1 << 40) - 1, 2**63): (1, 1)}  # unit * batch beyond 2^64
     assert ask([("makes_two", *c) for c in cases]) == [m for m, _ in cases.values()]
     assert ask([("runs_two", *c) for c in cases]) == [r for _, r in cases.values()]
+
+
+# (log2 points, own columns, tiles per transform or image) -> transforms up to
+# which a launch on 256 CUs takes 4, 8, 16 columns (None: never)
+NARROW = {(8, 32, 8): (4, 32, 64), (8, 32, 16): (2, 16, 32), (9, 8, 32): (4, None, None), (8, 32, 32): (1, 8, 16),
+          (10, 16, 16): (4, 16, None), (9, 16, 64): (1, 8, None), (10, 16, 32): (2, 8, None), (10, 16, 64): (1, 4, None),
+          (7, 64, 256): (None, None, 1), (8, 32, 512): (None, None, 1), (7, 64, 16): (None, 8, 16), (9, 16, 32): (2, 16, None),
+          (11, 8, 2): (64, None, None), (12, 8, 8): (16, None, None)}
+
+
+def test_launches_short_of_workgroups_are_narrowed(ask):
+    for (log_l, g, tiles), limits in NARROW.items():
+        edges = [(w, n) for w, n in zip((4, 8, 16), limits) if n]
+        calls, want = [], []
+        for i, (w, n) in enumerate(edges):
+            calls += [("narrow", log_l, g, tiles * n, 256), ("narrow", log_l, g, tiles * (n + 1), 256)]
+            above = [v for v, m in edges[i + 1:] if m >= n + 1]
+            want += [w, above[0] if above else 0]
+        assert ask(calls) == want, (log_l, g, tiles)
+
+
+def test_narrow_forms_fit_their_kernels(ask):
+    # every width the rule can give: one that the kernel has (tile_narrows in
+    # kernels/fft_tile.hpp), a whole wave, no more threads than the kernel's bound
+    for log_l, g, per_thread in ((7, 64, 32), (8, 32, 32), (8, 16, 32), (9, 16, 32), (10, 16, 32), (11, 8, 32), (12, 8, 32), (9, 8, 16)):
+        got = set(ask([("narrow", log_l, g, t, cu) for t in list(range(1, 300)) + [512, 1024, 4096] for cu in (1, 32, 256, 304)]))
+        for w in got - {0}:
+            threads = (w << log_l) // 16
+            assert w in (4, 8, 16) and w < g and (log_l, g) != (8, 16)
+            assert threads % 64 == 0 and 64 <= threads <= (g << log_l) // per_thread
+            # the launch steps tiles by g / w of the pass's own (FftPlan::run)
+            assert g % w == 0
