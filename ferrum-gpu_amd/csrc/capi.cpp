@@ -35,8 +35,9 @@ struct fg_device {
     HipBackend::Module fft_module;
     std::mutex mu;  // guards the plan cache and the staging buffer of the host path
     // Host-path plans, key: (dims, log_n or log_cols, log_rows (0 for 1D), batch);
-    // the kCachedPlans most recently used are kept (a multi-pass plan holds up
-    // to a 128 MiB workspace, so the cache must not grow with every new batch).
+    // the kCachedPlans most recently used are kept (a multi-pass plan holds
+    // workspaces of up to the chunk limit, 256 MiB by default, so the cache
+    // must not grow with every new batch).
     struct CachedPlan {
         std::unique_ptr<FftPlan> plan;
         uint64_t last_use = 0;

@@ -234,11 +234,13 @@ bool use_halves_tile(uint32_t log_l, uint32_t g, bool rowwise) {
 }
 
 bool use_row_halves_tile(uint32_t log_l, uint32_t g, bool rowwise) {
-    // The 1D last pass of 512 / 1024 points in 16-row tiles: every row load
-    // of the tile is issued at once and each half of the positions is
-    // transposed through an LDS tile of L/2 positions, then the exchanges run
-    // in halves -- 34 / 68 KB instead of 68 / 136 KB, so four / two
-    // workgroups per CU instead of two / one.  Measured on gfx950 at 512 MiB
+    // The 1D last pass of 512 / 1024 points in 16-row tiles: every load of the
+    // tile is issued at once and the exchanges run in halves through an LDS
+    // tile of L/2 positions -- 34 / 68 KB instead of 68 / 136 KB, so four /
+    // two workgroups per CU instead of two / one (row_halves_direct in
+    // kernels/fft_tile.hpp: these load their Stockham positions and the first
+    // exchange turns the tile; 256 points load along the rows and turn each
+    // half through LDS first).  Measured on gfx950 at 512 MiB
     // per execution (two alternations, us): 2^20 397.7 / 396.9 -> 368.4 /
     // 369.9, 2^19 365.4 / 366.3 -> 362.3 / 362.7.  At 256 points (already
     // four workgroups per CU at 16 rows) halves of 16 rows gained nothing;
@@ -455,12 +457,14 @@ uint64_t split_narrow_limit(uint32_t log_l) {
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) {
     // A launch in the pass's own tiles of G columns that would leave CUs idle,
     // or hold them at less than one round of narrower tiles, takes the
-    // narrowest form (fft_tile_narrow; at least one wave per workgroup) whose
-    // workgroups are resident all at once: 1024 threads per CU (16 waves at
-    // the kernels' 128 VGPRs; the LDS allows as many), so 1024 / block of the
-    // pass's own blocks, which a narrow form of half the elements per thread
-    // equals per column; 4 columns, whose 32-byte pieces cost L2 requests,
-    // only up to one workgroup per CU.  Measured on gfx950, us per
+    // narrowest form (fft_tile_narrow; at least one wave per workgroup) of at
+    // most as many workgroups per CU as the pass's own tiles fit there: 1024
+    // threads (16 waves at the kernels' 128 VGPRs; the LDS allows as many) over
+    // their block.  A form of w = G / 2 columns has that block's size, so its
+    // limit is the residency; narrower ones have smaller blocks, of which more
+    // would fit, but lose before (2^16 x 48 and x 64 below: 8 columns are still
+    // resident and slower than 16).  4 columns, whose 32-byte pieces cost L2
+    // requests, only up to one workgroup per CU.  Measured on gfx950, us per
     // execution, own tiles / narrow by this rule (the passes of one plan
     // narrowed one at a time: 4, 8, 16 columns): first pass of 256 points,
     // 2^16 x 1 12.4 / 10.0 (8 columns 10.3), x 16 17.0 / 14.6 at 8, x 48 27.8
@@ -474,10 +478,10 @@ uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count) 
     // Not with two chunks in flight, where the other stream's launch fills the
     // CUs: 2^16 x 300 (a last chunk of 44 transforms) 104.3 -> 107.4.
     if (log_l == 8 && g == 16) return 0;  // the middle pass of 2^23 points and more (tile_narrows)
-    const uint64_t resident = (uint64_t)cu_count * (1024 / (g * ((1u << log_l) / 32)));  // for w >= 8
+    const uint64_t most = (uint64_t)cu_count * (1024 / (g * ((1u << log_l) / 32)));  // for w >= 8
     for (uint32_t w = 4; w < g && w <= 16; w *= 2) {
         if ((w << log_l) / 16 < 64) continue;
-        if (tiles * (g / w) <= (w == 4 ? (uint64_t)cu_count : resident)) return w;
+        if (tiles * (g / w) <= (w == 4 ? (uint64_t)cu_count : most)) return w;
     }
     return 0;
 }

@@ -40,10 +40,12 @@ KernelArtifact fft_code_object();
 constexpr uint32_t kMinLogN1D = 2, kMaxLogN1D = 24, kMaxLogNSingle = 15;
 constexpr uint32_t kMinLogN2D = 4, kMaxLogN2D = 12;
 // Complex elements from which a multi-launch plan's split-layout execution is
-// fused into its end passes (2^16 x 4, us: staged 20.2, fused 8.9).  Smaller
-// batches (2^16 x 3 and less, 2^17 x 1, 2D images up to 2^17 elements) would
-// gain as much, but keep the staged form: captured graphs of such calls hold
-// launches() + 2 nodes, which the suite counts.
+// fused into its end passes (2^16 x 4, us: staged 15.3, fused 9.2; 256 x 256 x 4
+// 15.3, 9.2).  It is no limit of speed: smaller batches gain as much (2^16 x 1
+// 14.9, 8.2, x 3 15.7, 9.3, 2^17 x 1 15.2, 9.3, 256 x 256 x 1 13.6, 8.2), but
+// keep the staged form, because captured graphs of such calls hold launches() +
+// 2 nodes and tests/test_gpu_runtime_fixes.py and tests/test_zz_no_alloc.py pin
+// that count.
 constexpr uint64_t kFusedSplitElems = 1u << 18;
 
 class FftPlan {
@@ -296,13 +298,14 @@ bool column_pass_loads_cached(uint32_t log_n, uint32_t last_g, uint64_t bytes, b
 // Bytes of a launch's split input up to which a first pass of 2^log_l points
 // may run in a narrow form.
 uint64_t split_narrow_limit(uint32_t log_l);
-// Columns per workgroup of a launch of `tiles` tiles of a pass (2^log_l points, g columns per tile) in its narrow form; 0: its own tiles.
+// Columns per workgroup of a launch of `tiles` tiles of a pass (2^log_l points,
+// g columns per tile) in its narrow form; 0: its own tiles.
 uint32_t narrow_width(uint32_t log_l, uint32_t g, uint64_t tiles, int cu_count);
 // Whether the column FFT of an image with 2^log_rows rows runs as two passes.
 bool split_2d_columns(uint32_t log_rows);
 // Largest chunk (bytes of one chunk's array) a multi-launch plan created from
 // now on runs with its intermediates cached: FERRUM_GPU_CHUNK_MIB at load, else
-// 128 MiB (half the 256 MB Infinity Cache).  0 = no chunking: one chunk of
+// 256 MiB (the Infinity Cache); two chunks in flight take half of it each.  0 = no chunking: one chunk of
 // the whole batch, every pass streaming.
 size_t chunk_limit_bytes();
 void set_chunk_limit_bytes(size_t bytes);

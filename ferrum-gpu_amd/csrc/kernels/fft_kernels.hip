@@ -366,8 +366,8 @@ extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
 // fg_tile_l<LOGL>_g<G>_<c|r|h>[_<policy>]: one pass over G columns of length
 // 2^LOGL per workgroup (G * 2^LOGL / 16 threads; 'h': / 32).  'c': columns
 // contiguous in memory (column passes); 'r': rows contiguous (the last 1D
-// pass, which transposes through LDS); 'h': a column pass with 32 elements
-// per thread and the exchanges in halves (the first 1D pass).  Policy (fft_common.hpp, gload/gstore): none =
+// pass, whose first exchange turns the tile); 'h', 'rh': the same passes with
+// 32 elements per thread and the exchanges in halves.  Policy (fft_common.hpp, gload/gstore): none =
 // stream in and out; _sc = stream in, cached out (a chunk's first pass); _cc
 // (middle passes); _cs = cached in, stream out (last pass).  The host picks
 // the names in fft_plan.cpp (tile_name).
@@ -433,9 +433,9 @@ FG_TILE_HALVES_P(8, 32, _cs, true, false)
 FG_TILE_HALVES_P(9, 16, _cs, true, false)
 FG_TILE_HALVES_P(10, 16, _cs, true, false)
 // 1D last passes of 256 points in 32-row tiles and of 512 / 1024 points in
-// 16-row tiles: rows in (all loads issued at once, each half transposed
-// through LDS), exchanges in halves, columns out (256- / 128-byte pieces),
-// streamed out or unchunked.
+// 16-row tiles: rows in (all loads issued at once; 256 points turn each half
+// through LDS, 512 and 1024 in the first exchange), exchanges in halves,
+// columns out (256- / 128-byte pieces), streamed out or unchunked.
 #define FG_TILE_ROW_HALVES(LOGL, G, TAG, LC, SC)                                                           \
     extern "C" __global__ __launch_bounds__(G * HalvesShape<LOGL>::T) __attribute__((amdgpu_waves_per_eu(4))) \
     void fg_tile_l##LOGL##_g##G##_rh##TAG(const float2* __restrict__ in, float2* __restrict__ out,             \

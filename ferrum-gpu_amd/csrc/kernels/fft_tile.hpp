@@ -266,11 +266,12 @@ __device__ __forceinline__ TileCoords tile_coords(const TileGeom& g) {
 // ROWWISE: input elements of a column are contiguous (ies == 1, rows of a
 // matrix): T consecutive lanes load a row's Stockham positions t0 + T*m (8*T
 // contiguous bytes per access) and the first exchange turns the tile
-// (RowTileStages).  Otherwise columns are contiguous (ics == 1) and consecutive lanes load consecutive
-// columns.  Output always has ocs == 1.
+// (RowTileStages).  Otherwise columns are contiguous (ics == 1) and consecutive
+// lanes load consecutive columns.  Output always has ocs == 1.
 // LOAD_CACHED / STORE_CACHED select the pass's cache policy (gload/gstore).
-// CONJ: the body reads the inverse's conjugation flags; forward passes
-// (flags == 0) run the CONJ = false body, which has no per-element selects.
+// CONJ: the body reads the inverse's conjugation flags; forward passes (no
+// FG_PASS_CONJ bit) run the CONJ = false body, which has no per-element
+// selects.
 // Global addresses are a wave-uniform row base (scalar registers) plus a
 // 32-bit per-lane byte offset, so each access costs no 64-bit vector
 // arithmetic; a tile's offsets stay below 2^32 bytes (one transform or image
@@ -341,10 +342,11 @@ __device__ __forceinline__ void fft_tile_body(const Src src, const Dst dst,
 //  * The cache-resident 1D middle pass of 256 points: 16 columns (whole
 //    128-byte lines) in 17 KB.
 //  * 1D last passes (ROWWISE: rows in, transposed store) of 256 points in
-//    32-row tiles and of 512 / 1024 points in 16-row tiles: every row load
-//    is issued at once and each half of the positions is transposed through
-//    the same L/2-position LDS tile, so 33 / 34 / 68 KB instead of the
-//    16-element tile's 66 / 68 / 136 KB.
+//    32-row tiles and of 512 / 1024 points in 16-row tiles: every load is
+//    issued at once and the tile is turned through the same L/2-position LDS
+//    tile (256 points: each half by itself; 512 and 1024: in the first
+//    exchange), so 34 / 34 / 68 KB instead of the 16-element tile's 66 / 68 /
+//    136 KB.
 //  * 2D column passes of 1024 .. 4096 points, narrow tiles (8 columns, the
 //    position-padded layout): twice the columns of the 16-element tile in the
 //    same LDS (136 KB at 4096 points), so 64-byte row pieces instead of 32.
@@ -576,7 +578,8 @@ constexpr int tile_narrow_lds() {
     return ROWWISE ? RowTileLayout<LOGL, W>::ELEMS : TileLayout<LOGL, W>::ELEMS;
 }
 
-// LDS of a halves pass: its own tile's, or a narrow form's (at most 3 % more).
+// LDS of a halves pass: its own tile's, or a narrow form's (up to 4 % more: 35072
+// bytes instead of 33792 for the 32-row tiles of 256 points).
 template <int LOGL, int G, bool ROWWISE>
 constexpr int tile_halves_lds() {
     int n = ROWWISE && row_halves_direct<LOGL>() ? RowTileLayout<LOGL - 1, G>::ELEMS : TileLayout<LOGL - 1, G>::ELEMS;

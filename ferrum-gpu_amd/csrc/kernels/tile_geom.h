@@ -23,12 +23,14 @@ namespace fg {
  * 0 for its own width. */
 #define FG_PASS_WIDTH_SHIFT 8
 
-/* Tile orders of narrow tiles (G < 16 columns: 128 / (8 G) tiles share each
- * 128-byte line).  Workgroups are dealt round-robin over the 8 XCDs, so
- * workgroup b runs on XCD b % 8 as that XCD's (b / 8)-th.
+/* Tile orders of tiles narrower than a 128-byte line: 16 columns of
+ * interleaved data, 32 of the split layout's f32 arrays (TileIn::LINE and its
+ * like in fft_tile.hpp), so LINE / G tiles share each line.  Workgroups are
+ * dealt round-robin over the 8 XCDs, so workgroup b runs on XCD b % 8 as that
+ * XCD's (b / 8)-th.
  *   XCD_RANGES: XCD x takes the contiguous tile range [x grid/8, (x+1) grid/8)
  *     (grid a multiple of 8);
- *   LINE_GROUPS: the groups of s = 16 / G tiles that share lines are dealt
+ *   LINE_GROUPS: the groups of s = LINE / G tiles that share lines are dealt
  *     round-robin over the XCDs: XCD x's j-th workgroup takes tile
  *     s (8 (j / s) + x) + j mod s (grid a multiple of 8 s), so the XCDs work
  *     on neighbouring line groups at the same time. */
