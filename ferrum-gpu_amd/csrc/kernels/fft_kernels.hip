@@ -466,8 +466,8 @@ FG_TILE_NARROW(9, 8, true, r)
 // layout's own limits (column_pass_loads_cached, split_narrow_limit in
 // fft_plan.cpp); last passes stream their stores from their own tiles of 16
 // columns and more, and store through the caches from narrow ones.  Measured
-// on gfx950 against the staged form, us: 2^18 x 16 63.8 -> 28.1, 2^16 x 64
-// 59.5 -> 24.2, 2^20 x 1 37.0 -> 18.6, 2^24 x 1 219 -> 136, 512 x 512 x 3 25.8
+// on gfx950 against the staged form, us: 2^18 x 16 63.8 -> 29.2, 2^16 x 64
+// 59.5 -> 25.4, 2^20 x 1 37.0 -> 18.6, 2^24 x 1 219 -> 136, 512 x 512 x 3 25.8
 // -> 12.2, 256 x 256 x 200 138.7 -> 67.3.
 #define FG_TILE_SPLIT_IN(LOGL, G)                                                                          \
     extern "C" __global__ __launch_bounds__(G * HalvesShape<LOGL>::T) __attribute__((amdgpu_waves_per_eu(4))) \
